@@ -19,19 +19,7 @@
 // L (16..256) and K (16..256) grow with the image so that small images get
 // short serial walks and many threads.  The mod-255 alpha channel uses sums
 // instead of maps.
-//
-// DITHER_FLOYDSTEINBERG (:1350-1412) diffuses a 12-bit error to the right
-// (7/16) and to the row below (3, 5 and the rest of the remainder).  Texel
-// (x, y) reads the accumulated error A_y[x+1] that row y-1 finalises when it
-// processes texel x+1, so rows form a wavefront with a skew of two texels:
-// thread r of one workgroup handles row y0 + r and at step t texel
-// x = t - 2r.  Each row keeps a window of its not yet final downward errors
-// in registers and hands A_{y+1}[x] to the next row through LDS (double
-// buffered by step parity); the last row of a band hands them to the first
-// row of the next band through a global carry row.  The reference reuses one
-// error buffer for the colour and the alpha pass and does not clear the
-// part the alpha pass reads for its first row: that row starts from the
-// red-channel errors the colour pass left there (see k_dither_fs).
+// DITHER_FLOYDSTEINBERG is in dither_fs.hip.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -248,151 +236,6 @@ __global__ void k_quantize_none(const uint8_t *__restrict__ src, int srccomps, l
 	}
 }
 
-// e7, e3, e5, e1 of floyd/floyd1 (:1227-1233), C division (toward zero)
-__device__ __forceinline__ void fs_split(int err, int &e7, int &e3, int &e5, int &e1)
-{
-	e7 = (err * 7 + 8) / 16;
-	err -= e7;
-	e3 = (err * 3 + 4) / 9;
-	err -= e3;
-	e5 = (err * 5 + 3) / 6;
-	err -= e5;
-	e1 = err;
-}
-
-// ---- Floyd-Steinberg ----
-// Rows per band R (the workgroup size) is a template parameter: 256, 512 or
-// 1024, the smallest that covers min(h, 1024).  The wavefront takes
-// ceil(h / R) * (w + 2R - 1) steps, each a dependent chain of about fifty
-// instructions plus an LDS hand-off and a barrier, so tall bands cut the
-// step count (a 4096^2 image: 24,572 steps at R = 1024 against 73,712 at 256).
-
-struct FsChan {
-	int off;    // byte offset of the channel in a source texel
-	int kind;   // 0: floyd(shift), 1: floyd1
-	int shift;
-};
-
-__device__ __forceinline__ int fs_load(const int *p)
-{
-	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void fs_store(int *p, int v)
-{
-	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// One Floyd-Steinberg pass per workgroup: workgroup k runs channel k
-// (c0, c1, c2) with its own carry row at carry + k * (w + 2); the channels
-// of the reference's colour pass are independent (separate error rows,
-// s2tc_algorithm.cpp:1356-1372), so they run side by side on different CUs.
-// init0 (w+2 ints, may be null) is A_0 of workgroup 0's channel, the errors
-// its first row starts from (zero otherwise).  rleft (w+2 ints, may be null)
-// receives what the reference's buffer holds in the first w+2 ints after the
-// pass, for workgroup 0's channel: the accumulated errors the last row read
-// (thisrow, when h-1 is even) or that row's downward errors (downrow, when
-// h-1 is odd).  The quantized step divides by maxval (15, 31 or 63) with one
-// high multiply: floor(v / d) = mul_hi(v, floor(2^32 / d) + 1) for v < 2^20
-// and odd d < 2^12, since the product overshoots v / d by less than
-// 2^-12 < 1 / d.
-template <int FS_R>
-__global__ __launch_bounds__(FS_R) void k_dither_fs(const uint8_t *__restrict__ src, int srccomps, int w, int h,
-                                                    FsChan c0, FsChan c1, FsChan c2, const int *__restrict__ init0,
-                                                    int *__restrict__ carry_all, int *__restrict__ rleft_all,
-                                                    uint8_t *__restrict__ out)
-{
-	__shared__ int slot[FS_R][2];
-	const int k = (int)blockIdx.x;
-	const FsChan ch = k == 0 ? c0 : k == 1 ? c1 : c2;
-	const int r = (int)threadIdx.x;
-	const int pw = w + 2;
-	int *carry = carry_all + (size_t)k * pw;
-	const int *init = k == 0 ? init0 : nullptr;
-	int *rleft = k == 0 ? rleft_all : nullptr;
-	const int maxval = (1 << (8 - ch.shift)) - 1;
-	const uint32_t rec = 0xffffffffu / (uint32_t)maxval + 1u;
-	for (int j = r; j < pw; j += FS_R) fs_store(&carry[j], init ? init[j] : 0);
-	__syncthreads();
-	for (int y0 = 0; y0 < h; y0 += FS_R) {
-		const int rows = min(FS_R, h - y0);
-		const int y = y0 + r;
-		const bool active = r < rows;
-		const uint8_t *srow = src + (size_t)(active ? y : 0) * (size_t)w * (size_t)srccomps + ch.off;
-		uint8_t *orow = out + (size_t)(active ? y : 0) * (size_t)w * 4 + ch.off;
-		int right = 0, win1 = 0, win2 = 0;
-		const int steps = w + 2 * (rows - 1) + 1;
-		for (int t = 0; t < steps; ++t) {
-			const int x = t - 2 * r;
-			if (active && x >= 0 && x <= w) {
-				int fin;
-				if (x < w) {
-					const int above = r == 0 ? fs_load(&carry[x + 1]) : slot[r - 1][(t - 1) & 1];
-					const int acc = above + right;
-					const int sv = srow[x * srccomps];
-					const int v = ((sv << 4) | (sv >> 4)) + acc;
-					int q, err;
-					if (ch.kind == 1) {
-						q = v >= 2048 ? 1 : 0;
-						err = v - (q ? 4095 : 0);
-					} else {
-						q = v >> (ch.shift + 4);
-						q = q < 0 ? 0 : (q > maxval ? maxval : q);
-						err = v - (int)__umulhi((uint32_t)(q * 4095), rec);
-					}
-					orow[x * 4] = (uint8_t)q;
-					int e7, e3, e5, e1;
-					fs_split(err, e7, e3, e5, e1);
-					right = e7;
-					fin = win1 + e3;
-					win1 = win2 + e5;
-					win2 = e1;
-					if (rleft && y == h - 1 && ((h - 1) & 1) == 0) rleft[x + 1] = acc;
-				} else {
-					fin = win1;
-				}
-				if (r + 1 < rows) slot[r][t & 1] = fin;  // A_{y+1}[x] for row y+1
-				else fs_store(&carry[x], fin);
-				if (rleft && y == h - 1 && ((h - 1) & 1) == 1) rleft[x] = fin;
-			}
-			__syncthreads();
-		}
-	}
-}
-
-template <int FS_R>
-static void fs_pass(int nch, const uint8_t *src, int srccomps, int w, int h, FsChan c0, FsChan c1, FsChan c2,
-                    const int *init0, int *carry, int *rleft, uint8_t *out, hipStream_t st)
-{
-	k_dither_fs<FS_R><<<nch, FS_R, 0, st>>>(src, srccomps, w, h, c0, c1, c2, init0, carry, rleft, out);
-}
-
-static int launch_rgb565_fs(const uint8_t *src, int srccomps, int w, int h, int alphabits, uint8_t *out,
-                            void *d_scratch, hipStream_t st)
-{
-	int *carry = (int *)d_scratch;          // 3 * (w + 2)
-	int *rleft = carry + 3 * (w + 2);        // w + 2
-	const bool alpha_fs = srccomps == 4 && (alphabits == 1 || alphabits == 4);
-	const FsChan cr{0, 0, 3}, cg{1, 0, 2}, cb{2, 0, 3};
-	const int R = h <= 256 ? 256 : h <= 512 ? 512 : 1024;
-	int *rl = alpha_fs ? rleft : nullptr;
-	// r, g and b: three workgroups, one channel each
-	if (R == 256) fs_pass<256>(3, src, srccomps, w, h, cr, cg, cb, nullptr, carry, rl, out, st);
-	else if (R == 512) fs_pass<512>(3, src, srccomps, w, h, cr, cg, cb, nullptr, carry, rl, out, st);
-	else fs_pass<1024>(3, src, srccomps, w, h, cr, cg, cb, nullptr, carry, rl, out, st);
-	if (int r = hip_check(hipGetLastError(), "dither FS colour kernel")) return r;
-	if (alpha_fs) {
-		// alpha starts from what the r pass left in the shared buffer
-		const FsChan ca{3, alphabits == 1 ? 1 : 0, 8 - alphabits};
-		if (R == 256) fs_pass<256>(1, src, srccomps, w, h, ca, ca, ca, rleft, carry, nullptr, out, st);
-		else if (R == 512) fs_pass<512>(1, src, srccomps, w, h, ca, ca, ca, rleft, carry, nullptr, out, st);
-		else fs_pass<1024>(1, src, srccomps, w, h, ca, ca, ca, rleft, carry, nullptr, out, st);
-		return hip_check(hipGetLastError(), "dither FS alpha kernel");
-	}
-	const long long n = (long long)w * h;
-	k_quantize_none<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(src, srccomps, n, alphabits, 0, 1, out);
-	return hip_check(hipGetLastError(), "quantize alpha kernel");
-}
-
 // ---- host launchers ----
 
 // Chunk length L and super chunk size K for n texels: powers of two with
@@ -427,18 +270,15 @@ static void simple_chunking(long long n, DChans &cs)
 	cs.stride = c.stride;
 }
 
-// scratch bytes of one dither mode: SIMPLE maps of up to four channels, FS
-// carry rows of three channels plus the row handed to the alpha pass
+// scratch bytes of SIMPLE: the maps of up to four channels
 static constexpr size_t simple_scratch_bytes(long long n)
 {
 	return (size_t)(4 * simple_chunking_of(n > 0 ? n : 1).stride + 256);
 }
-static constexpr size_t fs_scratch_bytes(int w) { return (size_t)(4 * ((long long)w + 2)) * sizeof(int) + 256; }
-
-size_t rgb565_scratch_bytes(int w, int h)
+size_t rgb565_scratch_bytes(int w, int h, int dither)
 {
-	const size_t simple = simple_scratch_bytes((long long)w * h), fs = fs_scratch_bytes(w);
-	return simple > fs ? simple : fs;
+	if (dither == DITHER_FLOYDSTEINBERG) return rgb565_fs_scratch_bytes(w, h);
+	return simple_scratch_bytes((long long)w * h);
 }
 
 static int run_simple(const uint8_t *src, int srccomps, long long n, DChans cs, uint8_t *out, uint8_t *scr,

@@ -253,7 +253,7 @@ static int encode_host_bands(Ctx *c, int srccomps, int width, int height, const 
 	const bool fused = dither == DITHER_NONE && srccomps == 4;
 	if (!fused) {
 		if (int r = c->q.ensure(n * 4)) return r;
-		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, brows) + 256)) return r;
+		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, brows, dither) + 256)) return r;
 	}
 	if (!c->copy_stream)
 		if (int r = hip_check(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking), "hipStreamCreate"))
@@ -275,7 +275,7 @@ static int encode_host_bands(Ctx *c, int srccomps, int width, int height, const 
 	if (!c->dither_ev)
 		if (int r = hip_check(hipEventCreateWithFlags(&c->dither_ev, hipEventDisableTiming), "hipEventCreate"))
 			return r;
-	uint8_t *carry = (uint8_t *)c->scratch.p + rgb565_scratch_bytes(width, brows);
+	uint8_t *carry = (uint8_t *)c->scratch.p + rgb565_scratch_bytes(width, brows, dither);
 	int next = 0;
 	auto on_chunk = [&](size_t uploaded) -> int {
 		bool waited = false;
@@ -370,7 +370,7 @@ static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, con
 			a.src_kind = S2TC_SRC_RGBA8;
 		} else {
 			if (int r = c->q.ensure(n * 4)) return r;
-			if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height))) return r;
+			if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height, dither))) return r;
 			if (int r = launch_rgb565(c->src.p, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p,
 			                          c->stream))
 				return r;
@@ -542,7 +542,7 @@ void rgb565_image(unsigned char *out, const unsigned char *rgba, int w, int h, i
 	const size_t n = (size_t)w * h;
 	int r = c->src.ensure(n * sc);
 	if (!r) r = c->q.ensure(n * 4);
-	if (!r) r = c->scratch.ensure(rgb565_scratch_bytes(w, h));
+	if (!r) r = c->scratch.ensure(rgb565_scratch_bytes(w, h, (int)dither));
 	if (!r) r = upload(c, c->src.p, rgba, n * sc);
 	if (!r) r = launch_rgb565(c->src.p, sc, w, h, alphabits, (int)dither, c->q.p, c->scratch.p, c->stream);
 	if (!r) r = hip_check(hipMemcpyAsync(out, c->q.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
