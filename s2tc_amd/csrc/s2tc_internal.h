@@ -45,13 +45,13 @@ int launch_encode(const EncodeArgs &a, hipStream_t stream, void *ext_scratch = n
 
 // rgb565_image on the device (dither.hip); d_scratch holds
 // rgb565_scratch_bytes(w, h, dither).
-// d_carry (4 bytes, NONE and SIMPLE only): the image is a band of rows of a
-// larger one; SIMPLE starts from the error state in d_carry when carry_in is
-// set (else from the reference's initial state) and leaves its end state
-// there for the next band.
+// d_carry_in / d_carry_out (4 bytes each, apart; SIMPLE only): the image is a
+// band of rows of a larger one, which starts from the error states in
+// d_carry_in (null: from the reference's initial ones) and leaves its end
+// states in d_carry_out for the next band.
 size_t rgb565_scratch_bytes(int w, int h, int dither);
 int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, int dither, void *d_out,
-                  void *d_scratch, hipStream_t st, void *d_carry = nullptr, int carry_in = 0);
+                  void *d_scratch, hipStream_t st, const void *d_carry_in = nullptr, void *d_carry_out = nullptr);
 
 // The Floyd-Steinberg dither (dither_fs.hip), arguments normalised.
 size_t rgb565_fs_scratch_bytes(int w, int h);

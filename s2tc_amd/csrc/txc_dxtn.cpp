@@ -298,7 +298,8 @@ static int encode_host_bands(Ctx *c, int srccomps, int width, int height, const 
 			} else {
 				uint8_t *bq = (uint8_t *)c->q.p + (size_t)r0 * width * 4;
 				if (int r = launch_rgb565(bsrc, srccomps, width, rows, alphabits, dither, bq, c->scratch.p,
-				                          c->dither_stream, carry, next > 0))
+				                          c->dither_stream, next > 0 ? carry + 4 * (next & 1) : nullptr,
+				                          carry + 4 * ((next + 1) & 1)))
 					return r;
 				if (int r = hip_check(hipEventRecord(c->dither_ev, c->dither_stream), "hipEventRecord")) return r;
 				if (int r = hip_check(hipStreamWaitEvent(c->stream, c->dither_ev, 0), "hipStreamWaitEvent")) return r;
