@@ -14,6 +14,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
 #include "s2tc_internal.h"
 
 namespace s2tc {
@@ -122,6 +126,62 @@ __global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ bloc
 	}
 }
 
+// ---- the sums of s2tc_amd_colordist_error ----
+
+// A call's pinned words for the workgroups' sums, kept for later calls on the
+// same device (allocating and clearing a device word took 25 us a call).  A
+// call owns its buffer from acquire to release, so calls from several threads
+// or on several streams do not meet.
+static const unsigned kSumsMax = 512;
+struct SumBuf {
+	int dev;
+	long long *sums, *dev_sums;  // [kSumsMax]
+};
+
+static std::mutex g_sum_mu;
+static std::vector<SumBuf *> g_sums;
+static const size_t kSumBufsKept = 16;
+
+static int sum_acquire(SumBuf **out)
+{
+	int dev = 0;
+	if (int r = hip_check(hipGetDevice(&dev), "hipGetDevice")) return r;
+	{
+		std::lock_guard<std::mutex> lk(g_sum_mu);
+		for (size_t i = 0; i < g_sums.size(); ++i)
+			if (g_sums[i]->dev == dev) {
+				*out = g_sums[i];
+				g_sums[i] = g_sums.back();
+				g_sums.pop_back();
+				return 0;
+			}
+	}
+	SumBuf *b = new SumBuf{dev, nullptr, nullptr};
+	int rc = hip_check(hipHostMalloc((void **)&b->sums, kSumsMax * sizeof(long long), hipHostMallocMapped),
+	                   "hipHostMalloc");
+	if (!rc) rc = hip_check(hipHostGetDevicePointer((void **)&b->dev_sums, b->sums, 0), "hipHostGetDevicePointer");
+	if (rc) {
+		if (b->sums) (void)hipHostFree(b->sums);
+		delete b;
+		return rc;
+	}
+	*out = b;
+	return 0;
+}
+
+static void sum_release(SumBuf *b)
+{
+	{
+		std::lock_guard<std::mutex> lk(g_sum_mu);
+		if (g_sums.size() < kSumBufsKept) {
+			g_sums.push_back(b);
+			return;
+		}
+	}
+	(void)hipHostFree(b->sums);
+	delete b;
+}
+
 }  // namespace s2tc
 
 using namespace s2tc;
@@ -163,16 +223,21 @@ extern "C" int s2tc_amd_colordist_error(const void *d_src, int src_kind, int wid
 	const int bw = (width + 3) / 4, bh = (height + 3) / 4;
 	if (bh > 4 * 65535) return set_error(S2TC_E_RANGE, "colordist_error: image too tall");
 	hipStream_t st = (hipStream_t)stream;
-	long long *d_sum = nullptr;
-	int rc = hip_check(hipMalloc((void **)&d_sum, sizeof(long long)), "hipMalloc");
-	if (!rc) rc = hip_check(hipMemsetAsync(d_sum, 0, sizeof(long long), st), "hipMemsetAsync");
+	SumBuf *b = nullptr;
+	if (int r = sum_acquire(&b)) return r;
+	const long long tiles = (long long)((bw + 63) / 64) * ((bh + 3) / 4);
+	// two workgroups per CU hide each other's loads
+	const unsigned grid = (unsigned)std::min<long long>(tiles, kSumsMax);
+	void *args[] = {(void *)&d_src, (void *)&width, (void *)&height, (void *)&d_blocks, (void *)&b->dev_sums};
+	int rc = hip_check(hipLaunchKernel(k, dim3(grid), dim3(64, 4), args, 0, st), "launch colour-distance kernel");
+	// also after a failed launch: nothing may still write to the buffer
+	const int rs = hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
+	if (!rc) rc = rs;
 	if (!rc) {
-		void *args[] = {(void *)&d_src, (void *)&width, (void *)&height, (void *)&d_blocks, (void *)&d_sum};
-		dim3 grid((unsigned)((bw + 63) / 64), (unsigned)((bh + 3) / 4)), block(64, 4);
-		rc = hip_check(hipLaunchKernel(k, grid, block, args, 0, st), "launch colour-distance kernel");
+		long long sum = 0;
+		for (unsigned i = 0; i < grid; ++i) sum += b->sums[i];
+		*total = sum;
 	}
-	if (!rc) rc = hip_check(hipMemcpyAsync(total, d_sum, sizeof(long long), hipMemcpyDeviceToHost, st), "D2H");
-	if (!rc) rc = hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
-	if (d_sum) (void)hipFree(d_sum);
+	sum_release(b);
 	return rc;
 }
