@@ -87,14 +87,12 @@ S2TC_D bool eval_color(int n0, uint32_t s0, int n1, uint32_t s1, uint32_t &c0, u
 {
 	if (!n0 && !n1) return false;
 	if (n0) {
-		int r = rmean((int)(s0 & 1023u), n0) & 31, g = rmean((int)((s0 >> 10) & 2047u), n0) & 63,
-		    b = rmean((int)(s0 >> 21), n0) & 31;
-		c0 = (uint32_t)((r << 11) | (g << 5) | b);
+		const Mean m(n0);
+		c0 = (m.of(s0 & 1023u) << 11) | (m.of((s0 >> 10) & 2047u) << 5) | m.of(s0 >> 21);
 	}
 	if (n1) {
-		int r = rmean((int)(s1 & 1023u), n1) & 31, g = rmean((int)((s1 >> 10) & 2047u), n1) & 63,
-		    b = rmean((int)(s1 >> 21), n1) & 31;
-		c1 = (uint32_t)((r << 11) | (g << 5) | b);
+		const Mean m(n1);
+		c1 = (m.of(s1 & 1023u) << 11) | (m.of((s1 >> 10) & 2047u) << 5) | m.of(s1 >> 21);
 	}
 	return true;
 }
@@ -148,8 +146,8 @@ S2TC_D uint64_t alpha_try_lane(const uint32_t (&tx)[16], const Masks &mk, int a0
 S2TC_D bool eval_alpha(int n0, int s0, int n1, int s1, int &a0, int &a1)
 {
 	if (!n0 && !n1) return false;
-	if (n0) a0 = rmean(s0, n0) & 255;
-	if (n1) a1 = rmean(s1, n1) & 255;
+	if (n0) a0 = (int)Mean(n0).of((uint32_t)s0);
+	if (n1) a1 = (int)Mean(n1).of((uint32_t)s1);
 	return true;
 }
 

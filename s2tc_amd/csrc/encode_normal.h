@@ -7,12 +7,13 @@
 //
 // Work split:
 //  * candidate gather: ballot + prefix count gives each opaque texel its
-//    position in the reference's candidate list (:940-951);
+//    position in the reference's candidate list (:940-951); a candidate word
+//    is colour | alpha << 16 | cell of the colour box << 24;
 //  * random candidates: lane t draws candidates t, t+16, ... with the
 //    counter-based generator (s2tc_prng.h) in the reference's draw order;
 //  * distance matrix: lane t computes rows i = 16p + t of dists[i][k]
-//    (:373-392): the first two row blocks into its registers, the rest
-//    into LDS;
+//    (:373-392): the first RB row blocks into its registers, the
+//    rest into LDS;
 //  * pair scan (reduce_colors_inplace, :393-410): for every row-block pair
 //    (p, q) lane t keeps its row of block p and its row of block q in
 //    registers and meets the 16 rows of block q by rotating them through the
@@ -27,7 +28,7 @@
 #pragma once
 
 #include "encode_fast.h"
-#include "kernel_table.h"  // S2TC_REG_RB
+#include "kernel_table.h"  // S2TC_RB_FEW and the sizes of the group memory
 
 namespace s2tc {
 
@@ -123,17 +124,16 @@ template <int END, bool DIAG, int PASS, bool NEG> struct ScanSteps<END, END, DIA
 	static S2TC_D void run(const int (&)[16], const int (&)[16], int, int, int, int, int, ScanKey &) {}
 };
 
-// The first S2TC_REG_RB row blocks of a block's distance matrix stay in the
-// registers of their lanes (RegRows); the row memory holds the rows from
-// 16 S2TC_REG_RB on.  Fewer rows in LDS let more workgroups share a CU.
-struct RegRows {
-	int r[S2TC_REG_RB][16];
+// The first RB row blocks of a block's distance matrix stay in the registers
+// of their lanes; the row memory holds the rows from 16 RB on.
+template <int RB> struct RegRows {
+	int r[RB][16];
 };
 
-// Row r >= 16 S2TC_REG_RB from the row memory.
-S2TC_D void load_row(const int *rows, int r, int (&X)[16])
+// Row r >= 16 RB from the row memory.
+template <int RB> S2TC_D void load_row(const int *rows, int r, int (&X)[16])
 {
-	const int4 *p = (const int4 *)(rows + (r - 16 * S2TC_REG_RB) * S2TC_RS);
+	const int4 *p = (const int4 *)(rows + (r - 16 * RB) * S2TC_RS);
 #pragma unroll
 	for (int k = 0; k < 4; ++k) {
 		int4 v = p[k];
@@ -145,29 +145,29 @@ S2TC_D void load_row(const int *rows, int r, int (&X)[16])
 }
 
 // Lane t's row of row block p (row 16p + t), wherever it lives.
-S2TC_D void get_rows(const int *rows, const RegRows &R, int p, int t, int (&X)[16])
+template <int RB> S2TC_D void get_rows(const int *rows, const RegRows<RB> &R, int p, int t, int (&X)[16])
 {
-	if (p >= S2TC_REG_RB) {
-		load_row(rows, 16 * p + t, X);
+	if (p >= RB) {
+		load_row<RB>(rows, 16 * p + t, X);
 		return;
 	}
 #pragma unroll
-	for (int z = 0; z < S2TC_REG_RB; ++z)
+	for (int z = 0; z < RB; ++z)
 		if (p == z) {
 #pragma unroll
 			for (int k = 0; k < 16; ++k) X[k] = R.r[z][k];
 		}
 }
-S2TC_D void put_rows(int *rows, RegRows &R, int p, int t, const int (&dv)[16])
+template <int RB> S2TC_D void put_rows(int *rows, RegRows<RB> &R, int p, int t, const int (&dv)[16])
 {
-	if (p >= S2TC_REG_RB) {
-		int4 *rp = (int4 *)(rows + (16 * p + t - 16 * S2TC_REG_RB) * S2TC_RS);
+	if (p >= RB) {
+		int4 *rp = (int4 *)(rows + (16 * p + t - 16 * RB) * S2TC_RS);
 #pragma unroll
 		for (int k = 0; k < 4; ++k) rp[k] = make_int4(dv[4 * k], dv[4 * k + 1], dv[4 * k + 2], dv[4 * k + 3]);
 		return;
 	}
 #pragma unroll
-	for (int z = 0; z < S2TC_REG_RB; ++z)
+	for (int z = 0; z < RB; ++z)
 		if (p == z) {
 #pragma unroll
 			for (int k = 0; k < 16; ++k) R.r[z][k] = dv[k];
@@ -175,8 +175,8 @@ S2TC_D void put_rows(int *rows, RegRows &R, int p, int t, const int (&dv)[16])
 }
 
 // Scan over all pairs i < j < m of the rows in LDS; pbw row blocks (uniform).
-template <int PASS, bool NEG>
-S2TC_D void pair_scan(const int *rows, const RegRows &R, int t, int m, int pbw, int qthr, ScanKey &st)
+template <int PASS, bool NEG, int RB>
+S2TC_D void pair_scan(const int *rows, const RegRows<RB> &R, int t, int m, int pbw, int qthr, ScanKey &st)
 {
 	for (int p = 0; p < pbw; ++p) {
 		int X[16];
@@ -290,10 +290,16 @@ template <int END, int KM> struct KeyStepsDiag<END, END, KM> {
 // offers its pair (first, second), whose sum is its row sum (min(x, x) = x).
 // Returns the winning pair order; best: the least sum (saturated at cap for
 // KEY_SAT), row-uniform like the order.
-template <int KM, bool MAP = false>
-S2TC_D uint32_t reduce_rows_key(const int *rows, const RegRows &R, int t, int m, int pbw, const uint32_t *ul,
+// HALF (m <= 8, pbw = 1): lanes 8..15 hold the rows of lanes 0..7 again, so that
+// four rotations meet every pair.
+template <int KM, bool MAP = false, bool HALF = false, int RB>
+S2TC_D uint32_t reduce_rows_key(const int *rows, const RegRows<RB> &R, int t, int m, int pbw, const uint32_t *ul,
                                 uint32_t cap, uint32_t &best)
 {
+	if (HALF) {
+		t &= 7;
+		pbw = 1;
+	}
 	typedef typename ScanKeyT<KM>::T K;
 	ScanKey st{0xffffffffu, 0xffffffffu, -1};
 	const auto orig = [&](uint32_t a) -> uint32_t { return MAP ? (ul[3 * a] & 0xffffu) : a; };
@@ -304,7 +310,7 @@ S2TC_D uint32_t reduce_rows_key(const int *rows, const RegRows &R, int t, int m,
 		const bool irow = i < m;
 		{
 			K kmin = ~(K)0;
-			KeyStepsDiag<1, 9, KM>::run(X, t, irow ? (uint32_t)t : 0xffffffffu, cap, kmin);
+			KeyStepsDiag<1, HALF ? 5 : 9, KM>::run(X, t, irow ? (uint32_t)t : 0xffffffffu, cap, kmin);
 			const uint32_t b = (uint32_t)(kmin & 15u), tt = (uint32_t)t;
 			const uint32_t lo = 16u * p + min(tt, b), hi = 16u * p + max(tt, b);
 			const bool ok = irow && key_valid<KM>(kmin);
@@ -333,8 +339,8 @@ S2TC_D uint32_t reduce_rows_key(const int *rows, const RegRows &R, int t, int m,
 // reduce_colors_inplace / _2fixpoints argmin over the rows: returns the
 // winning pair order i << 16 | j (group-uniform).  Candidate indices stay
 // below 2^15 (S2TC_MAX_NRANDOM), so every order is a positive int.
-template <bool NEG>
-S2TC_D uint32_t reduce_rows(const int *rows, const RegRows &R, int t, int m, int pbw)
+template <bool NEG, int RB>
+S2TC_D uint32_t reduce_rows(const int *rows, const RegRows<RB> &R, int t, int m, int pbw)
 {
 	ScanKey st{0xffffffffu, 0xffffffffu, -1};
 	pair_scan<1, NEG>(rows, R, t, m, pbw, -1, st);
@@ -351,30 +357,31 @@ S2TC_D uint32_t reduce_rows(const int *rows, const RegRows &R, int t, int m, int
 	return st.lo;
 }
 
-// Per-group LDS: rows 16 S2TC_REG_RB .. mc - 1 (the first row blocks stay in
-// registers), the
-// features of the first 16 candidates (the columns of every row), candidates
-// (565 | alpha << 16).  A row's own candidate feature is computed by its
+// Per-group LDS: the row memory (`ints` of it), the features of the first 16
+// candidates (the columns of every row), candidates (colour | alpha << 16 |
+// cell << 24).  A row's own candidate feature is computed by its
 // lane.  normal_group_smem (kernel_table.h) gives the host the same size for
 // a four-block workgroup.
 template <int CD> struct GroupSmem {
 	uint32_t *cand;
 	typename Dist<CD>::F *feat;
 	int *rows;
+	int ints;
 };
 
-template <int CD> S2TC_D size_t group_smem_bytes(int mc)
+template <int CD, int RB> S2TC_D size_t group_smem_bytes(int mc)
 {
-	return (size_t)mc * sizeof(uint32_t) + (size_t)max(mc - 16 * S2TC_REG_RB, 0) * S2TC_RS * sizeof(int) +
+	return (size_t)mc * sizeof(uint32_t) + (size_t)normal_row_ints(mc >> 4, RB) * sizeof(int) +
 	       16 * sizeof(typename Dist<CD>::F);
 }
 
-template <int CD> S2TC_D GroupSmem<CD> group_smem(uint8_t *base, int g, int mc)
+template <int CD, int RB> S2TC_D GroupSmem<CD> group_smem(uint8_t *base, int g, int mc)
 {
-	uint8_t *p = base + (size_t)g * group_smem_bytes<CD>(mc);
-	const size_t rb = (size_t)max(mc - 16 * S2TC_REG_RB, 0) * S2TC_RS * sizeof(int);
+	uint8_t *p = base + (size_t)g * group_smem_bytes<CD, RB>(mc);
+	const size_t rb = (size_t)normal_row_ints(mc >> 4, RB) * sizeof(int);
 	GroupSmem<CD> s;
 	s.rows = (int *)p;
+	s.ints = normal_row_ints(mc >> 4, RB);
 	s.feat = (typename Dist<CD>::F *)(p + rb);
 	s.cand = (uint32_t *)(p + rb + 16 * sizeof(typename Dist<CD>::F));
 	return s;
@@ -422,14 +429,12 @@ S2TC_D uint32_t color_refine_group(uint32_t tex, bool valid, const typename Dist
 		const uint32_t a0s = atot - a1, g0s = gtot - g1;
 		bool ok = (n0 | n1) != 0;
 		if (n0) {
-			int r = rmean((int)(a0s & 1023u), n0) & 31, g = rmean((int)g0s, n0) & 63,
-			    bb = rmean((int)((a0s >> 10) & 1023u), n0) & 31;
-			n0v = (uint32_t)((r << 11) | (g << 5) | bb);
+			const Mean mn(n0);
+			n0v = (mn.of(a0s & 1023u) << 11) | (mn.of(g0s) << 5) | mn.of((a0s >> 10) & 1023u);
 		}
 		if (n1) {
-			int r = rmean((int)(a1 & 1023u), n1) & 31, g = rmean((int)g1, n1) & 63,
-			    bb = rmean((int)((a1 >> 10) & 1023u), n1) & 31;
-			n1v = (uint32_t)((r << 11) | (g << 5) | bb);
+			const Mean mn(n1);
+			n1v = (mn.of(a1 & 1023u) << 11) | (mn.of(g1) << 5) | mn.of((a1 >> 10) & 1023u);
 		}
 		if (refine != REFINE_LOOP) {  // ALWAYS: take the evaluated endpoints unchecked
 			c0 = n0v;
@@ -499,8 +504,8 @@ S2TC_D uint32_t alpha_refine_group(int a, bool valid, int refine, int &a0, int &
 		a0 = na0;
 		a1 = na1;
 		const int n0 = (int)(c0p >> 13), n1 = (int)(c1p >> 13);
-		if (n0) na0 = rmean((int)(c0p & 8191u), n0) & 255;
-		if (n1) na1 = rmean((int)(c1p & 8191u), n1) & 255;
+		if (n0) na0 = (int)Mean(n0).of(c0p & 8191u);
+		if (n1) na1 = (int)Mean(n1).of(c1p & 8191u);
 		if (refine != REFINE_LOOP) {
 			a0 = na0;
 			a1 = na1;
@@ -521,6 +526,27 @@ S2TC_D uint32_t alpha_refine_group(int a, bool valid, int refine, int &a0, int &
 	return idx;
 }
 
+// x % l for x < 2^31 and 1 <= l <= 256 by a multiplier m in [2^32 / l - 2,
+// 2^32 / l]: mul_hi falls short of x / l by less than 1 before its floor, so it
+// is the quotient or one less, and the remainder, below 2 l, only needs the low
+// bits of the product.  m is an estimate from below by the approximate
+// reciprocal (short by less than 2^13 / l) plus the quotient of its remainder,
+// which is at most one short itself.
+struct Modulo {
+	uint32_t l, m;
+	S2TC_D explicit Modulo(int l_) : l((uint32_t)l_)
+	{
+		const float r = __builtin_amdgcn_rcpf((float)l_);
+		const uint32_t q = (uint32_t)(r * 4294963200.0f);  // 2^32 (1 - 2^-20)
+		m = q + (uint32_t)__builtin_fmaf((float)~(q * l), r, -0.0009765625f);
+	}
+	S2TC_D uint32_t of(uint32_t x) const
+	{
+		const uint32_t r = (x - __umul24(__umulhi(x, m) & 0xffffffu, l)) & 0xffffffu;
+		return min(r, r - l);
+	}
+};
+
 // The whole MODE_NORMAL block on one DPP row.  tex: this lane's quantized
 // texel (0 when outside the block), t: lane within the row (texel x-major
 // index), pbw: row blocks = ceil((16 + max(nrandom, 0)) / 16) (kernel-uniform),
@@ -540,7 +566,17 @@ template <int CD> struct PlainScan {
 // (first A, second A), whose sum is A's row sum.  Small colour boxes (smooth
 // blocks: the random candidates fall on few colours) shrink the scan from
 // m (m - 1) / 2 pairs to about u^2 / 2 for u distinct colours.
-template <int CD, bool DEDUP = false>
+//
+// The first two indices of every cell of the colour box (at most 256, where
+// the row memory holds the tables) are kept by atomic minima, entered as the
+// candidates are made; the list of first occurrences goes to the last 3 m ints
+// of the row memory.  Up to 16 cells, a lane has one cell and its place in the
+// list is the count of cells with an earlier first index; up to 8 colours in
+// all four blocks, the rows are held twice and four rotations do.  The kernel
+// is bound by vector instructions.  Measured (MI355X, 4096 x 4096 smooth normal
+// map, 64 random colours, LOOP): 501 us, 802 us with three passes over the
+// candidates for the list and two register row blocks.
+template <int CD, int RB, bool DEDUP>
 S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int nrandom, int refine, uint32_t bkey,
                                 int pbw, const GroupSmem<CD> &sm, BlockOut &o)
 {
@@ -548,6 +584,9 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 	typedef typename D::F F;
 	const int lane = (int)(threadIdx.x & 63);
 	const int gshift = lane & 48;
+	// at least 137 registers, so at most three waves to a SIMD: with four, the
+	// twelve workgroups that a CU's LDS holds go 4, 4, 4 and 0
+	if (RB == S2TC_RB_MANY) asm volatile("" ::: "v136");
 	const int x = t >> 2, y = t & 3;
 	const bool valid = x < w && y < h;
 	const int alpha = texel_a(tex);
@@ -558,90 +597,116 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 	const uint32_t mask = (uint32_t)(__ballot(use) >> gshift) & 0xffffu;
 	const int pos = __builtin_popcount(mask & ((1u << t) - 1u));
 	int n = __builtin_popcount(mask);
-	if (use) sm.cand[pos] = v | ((uint32_t)alpha << 16);
 	const bool none = n == 0;
 	if (none) n = 1;
-	if (none && t == 0) sm.cand[0] = 0u;
-	// One colour among the candidates (the random ones are drawn inside the
-	// block colours' box, :962-993, so they share it): every pair the scan can
-	// pick has that colour, and the scan is skipped.  The same for DXT5 alpha,
-	// except where the last-miplevel hack pairs a lone texel with alpha 0.
-	const int vmin = row_min(use ? (int)v : 0xffff), vmax = row_max(use ? (int)v : 0);
-	const bool cuni = none || vmin == vmax;
-	bool auni = false;
-	int aone = 0;
-	if (dxt == DXT5) {
-		const int amin = row_min(use ? alpha : 255), amax = row_max(use ? alpha : 0);
-		auni = amin == amax && (nrandom > 0 || n >= 2);
-		aone = amin;
-	}
-	__syncthreads();
 	int m = n;
-	int minr = 0, ming = 0, minb = 0, lr = 1, lg = 1, lb = 1;  // the colour box of the random candidates
+	bool cuni;               // one colour among the candidates (see below)
+	uint32_t vone;           // that colour
+	bool auni = false;       // one alpha (DXT5)
+	int aone = 0;
+	int lr = 1, lg = 1, lb = 1;  // the colour box of the random candidates
+	bool dd = false;         // repeated colours are dropped from the colour scan (DEDUP)
+	uint32_t *ul = nullptr;
+	int V = 1;
+	const int cap = sm.ints;
 	if (nrandom > 0) {  // (:962-993)
-		int r = c_r(v), g = c_g(v), b = c_b(v);
-		minr = row_min(use ? r : 255), ming = row_min(use ? g : 255), minb = row_min(use ? b : 255);
+		const int r = c_r(v), g = c_g(v), b = c_b(v);
+		int minr = row_min(use ? r : 255), ming = row_min(use ? g : 255), minb = row_min(use ? b : 255);
 		int maxr = row_max(use ? r : 0), maxg = row_max(use ? g : 0), maxb = row_max(use ? b : 0);
-		int mina = row_min(use ? alpha : 255), maxa = row_max(use ? alpha : 0);
-		if (none) minr = ming = minb = maxr = maxg = maxb = mina = maxa = 0;
+		if (none) minr = ming = minb = maxr = maxg = maxb = 0;
 		lr = maxr - minr + 1, lg = maxg - ming + 1, lb = maxb - minb + 1;
-		const int la = maxa - mina + 1;
-		const int dpc = dxt == DXT5 ? 4 : 3;
-		// a channel whose range is one value takes it for every draw (draw % 1
-		// is 0): blocks of one colour (and of one alpha) skip those draws
-		for (int c = t; c < nrandom; c += 16) {
-			const uint32_t k = (uint32_t)(c * dpc);
-			uint32_t cr = (uint32_t)minr, cg = (uint32_t)ming, cb = (uint32_t)minb, ca = 0;
-			if (!cuni) {
-				cr += (uint32_t)s2tc_prng_draw(bkey, k) % (uint32_t)lr;
-				cg += (uint32_t)s2tc_prng_draw(bkey, k + 1) % (uint32_t)lg;
-				cb += (uint32_t)s2tc_prng_draw(bkey, k + 2) % (uint32_t)lb;
-			}
-			if (dxt == DXT5) {
-				ca = (uint32_t)mina;
-				if (la > 1) ca += (uint32_t)s2tc_prng_draw(bkey, k + 3) % (uint32_t)la;
-			}
-			sm.cand[n + c] = (cr << 11) | (cg << 5) | cb | (ca << 16);
+		V = mul_i24(mul_i24(lr, lg), lb);
+		cuni = V == 1;
+		vone = (uint32_t)((minr << 11) | (ming << 5) | minb);
+		int mina = 0, la = 1;
+		if (dxt == DXT5) {
+			mina = row_min(use ? alpha : 255);
+			int maxa = row_max(use ? alpha : 0);
+			if (none) mina = maxa = 0;
+			la = maxa - mina + 1;
+			auni = la == 1;
+			aone = mina;
 		}
 		m = n + nrandom;
-	} else if (n == 1) {  // "hack for last miplevel" (:996-1001); ca[1] pinned to 0
-		if (t == 0) sm.cand[1] = sm.cand[0] & 0xffffu;
-		n = m = 2;
+		int *T1 = sm.rows, *T2 = sm.rows + V;
+		if constexpr (DEDUP && PlainScan<CD>::value) {
+			dd = !cuni && V <= 256 && 2 * V + 3 * m <= cap;
+			ul = (uint32_t *)(sm.rows + cap - 3 * m);
+			if (dd)
+				for (int z = t; z < V; z += 16) T1[z] = T2[z] = 0x7fffffff;
+			__syncthreads();
+		}
+		// candidate i of cell z: the first two indices of every cell
+		const auto enter = [&](int z, int i) {
+			const int old = atomicMin(&T1[z], i);
+			if (old != 0x7fffffff) atomicMin(&T2[z], max(old, i));
+		};
+		const auto cell = [&](int cr, int cg, int cb) {
+			return DEDUP && PlainScan<CD>::value ? mad_i24(mad_i24(cr, lg, cg), lb, cb) : 0;
+		};
+		if (use) {
+			const int z = cell(r - minr, g - ming, b - minb);
+			sm.cand[pos] = v | ((uint32_t)alpha << 16) | ((uint32_t)z << 24);
+			if (dd) enter(z, pos);
+		}
+		if (none && t == 0) sm.cand[0] = 0u;
+		const int dpc = dxt == DXT5 ? 4 : 3;
+		// a channel whose range is one value takes it for every draw (draw % 1
+		// is 0): a wave skips the draws that no block of it needs
+		const bool anyr = __any(lr > 1), anyg = __any(lg > 1), anyb = __any(lb > 1), anya = __any(la > 1);
+		const Modulo mr(lr), mg(lg), mb(lb);
+		const Modulo ma(la);
+		for (int c = t; c < nrandom; c += 16) {
+			const uint32_t k = (uint32_t)(c * dpc);
+			uint32_t cr = 0, cg = 0, cb = 0, ca = (uint32_t)mina;
+			if (anyr) cr = mr.of((uint32_t)s2tc_prng_draw(bkey, k));
+			if (anyg) cg = mg.of((uint32_t)s2tc_prng_draw(bkey, k + 1));
+			if (anyb) cb = mb.of((uint32_t)s2tc_prng_draw(bkey, k + 2));
+			if (anya) ca += ma.of((uint32_t)s2tc_prng_draw(bkey, k + 3));
+			const int z = cell((int)cr, (int)cg, (int)cb);
+			sm.cand[n + c] = vone + (cr << 11) + (cg << 5) + cb + (ca << 16) + ((uint32_t)z << 24);
+			if (dd) enter(z, n + c);
+		}
+	} else {
+		const int vmin = row_min(use ? (int)v : 0xffff), vmax = row_max(use ? (int)v : 0);
+		cuni = none || vmin == vmax;
+		vone = none ? 0u : (uint32_t)vmin;
+		if (dxt == DXT5) {
+			const int amin = row_min(use ? alpha : 255), amax = row_max(use ? alpha : 0);
+			auni = amin == amax && n >= 2;
+			aone = amin;
+		}
+		if (use) sm.cand[pos] = v | ((uint32_t)alpha << 16);
+		if (none && t == 0) sm.cand[0] = 0u;
+		if (n == 1) {  // "hack for last miplevel" (:996-1001); ca[1] pinned to 0
+			__syncthreads();
+			if (t == 0) sm.cand[1] = sm.cand[0] & 0xffffu;
+			n = m = 2;
+		}
 	}
 	__syncthreads();
 
-	// Repeated colours (DEDUP).  In this block's row memory (16 (pbw -
-	// S2TC_REG_RB) rows of S2TC_RS ints): T1[V] and T2[V] over the colour box
-	// (V <= 256 cells) take
-	// the first and second candidate index of each colour by atomic minimum,
-	// then the list of first occurrences goes to the last 3 m ints, which the
-	// compacted rows (written from the top) must not reach.  Every lane of the
-	// workgroup passes the barriers; blocks that do not qualify skip the work.
 	int mu = m, pbu = pbw;
-	bool dd = false;
-	uint32_t *ul = nullptr;
 	if constexpr (DEDUP && PlainScan<CD>::value) {
-		const int cap = 16 * (pbw - S2TC_REG_RB) * S2TC_RS;
-		const int V = lr * lg * lb;
-		dd = !cuni && nrandom > 0 && pbw >= 2 && V <= 256 && 2 * V + 3 * m <= cap;
-		int *T1 = sm.rows, *T2 = sm.rows + V;
-		ul = (uint32_t *)(sm.rows + cap - 3 * m);
-		const auto cell = [&](uint32_t c) {
-			return ((c_r(c) - minr) * lg + (c_g(c) - ming)) * lb + (c_b(c) - minb);
-		};
-		if (dd)
-			for (int z = t; z < V; z += 16) T1[z] = T2[z] = 0x7fffffff;
-		__syncthreads();
-		if (dd)
-			for (int i = t; i < m; i += 16) atomicMin(&T1[cell(sm.cand[i] & 0xffffu)], i);
-		__syncthreads();
-		if (dd)
-			for (int i = t; i < m; i += 16) {
-				const int z = cell(sm.cand[i] & 0xffffu);
-				if (T1[z] != i) atomicMin(&T2[z], i);
+		const int *T1 = sm.rows, *T2 = sm.rows + V;
+		if (dd && V <= 16) {
+			// one cell per lane: its place in the list is the number of cells
+			// that come first earlier
+			const int f = t < V ? T1[t] : 0x7fffffff;
+			const int sec = t < V ? T2[t] : 0x7fffffff;
+			const bool have = f != 0x7fffffff;
+			mu = __builtin_popcount((uint32_t)(__ballot(have) >> gshift) & 0xffffu);
+			int rank = 0;
+#define S2TC_RANK(R) rank += dpp_i<0x120 + R>(f) < f ? 1 : 0;
+			S2TC_RANK(1) S2TC_RANK(2) S2TC_RANK(3) S2TC_RANK(4) S2TC_RANK(5) S2TC_RANK(6) S2TC_RANK(7) S2TC_RANK(8)
+			S2TC_RANK(9) S2TC_RANK(10) S2TC_RANK(11) S2TC_RANK(12) S2TC_RANK(13) S2TC_RANK(14) S2TC_RANK(15)
+#undef S2TC_RANK
+			if (have) {
+				ul[3 * rank] = (uint32_t)f | (sm.cand[f] << 16);
+				ul[3 * rank + 1] = sec == 0x7fffffff ? 0xffffffffu : (uint32_t)sec;
 			}
-		__syncthreads();
-		if (dd) {
+			pbu = 1;
+		} else if (dd) {
 			int base = 0;
 			for (int p = 0; p < pbw; ++p) {
 				const int i = 16 * p + t;
@@ -649,8 +714,8 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 				uint32_t c = 0u;
 				int sec = 0x7fffffff;
 				if (i < m) {
-					c = sm.cand[i] & 0xffffu;
-					const int z = cell(c);
+					c = sm.cand[i];
+					const int z = (int)(c >> 24);
 					first = T1[z] == i;
 					sec = T2[z];
 				}
@@ -664,9 +729,9 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 			}
 			mu = base;
 			pbu = (mu + 15) >> 4;
-			// the compacted rows (16 (pbu - S2TC_REG_RB) of them are stored)
+			// the compacted rows (16 (pbu - RB) of them are stored)
 			// must stay clear of the list, and must save work
-			if (pbu >= pbw || 16 * max(pbu - S2TC_REG_RB, 0) * S2TC_RS + 3 * m > cap) {
+			if (pbu >= pbw || 16 * max(pbu - RB, 0) * S2TC_RS + 3 * m > cap) {
 				dd = false;
 				mu = m;
 				pbu = pbw;
@@ -682,9 +747,11 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 	// dists[i][k] rows (:373-392): square part dist(c[min], c[max]), box part
 	// dist(c[i], c[k]); with DEDUP the rows of the list of first occurrences,
 	// each with its row sum.
-	RegRows R;
+	const bool half = DEDUP && PlainScan<CD>::value && __all((int)(cuni || (dd && mu <= 8)));
+	const bool whole = __all((int)(cuni || n == 16));
+	RegRows<RB> R;
 	for (int p = 0; p < (cuni ? 0 : pbu); ++p) {
-		const int i = 16 * p + t;
+		const int i = half ? t & 7 : 16 * p + t;
 		const bool irow = i < mu;
 		const F fi = D::feat(dd ? (irow ? ul[3 * i] >> 16 : 0u) : sm.cand[irow ? i : 0] & 0xffffu);
 		int dv[16];
@@ -694,7 +761,13 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 			int d;
 			if (IsSymmetric<CD>::value) d = D::d(fi, fk);
 			else d = (i < n && k < i) ? D::d(fk, fi) : D::d(fi, fk);
-			dv[k] = (irow && k < n) ? d : 0;
+			dv[k] = d;
+		}
+		// columns that are no candidates count nothing; rows that are none are
+		// never asked for
+		if (!whole) {
+#pragma unroll
+			for (int k = 0; k < 16; ++k) dv[k] = k < n ? dv[k] : 0;
 		}
 		put_rows(sm.rows, R, p, t, dv);
 		if (dd && irow) {
@@ -707,17 +780,19 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 	__syncthreads();
 	uint32_t c0, c1;
 	if (cuni) {
-		c0 = c1 = none ? 0u : (uint32_t)vmin;
+		c0 = c1 = vone;
 	} else {
 		uint32_t cbest, best;
 		if constexpr (DistBound<CD>::value != 0) {
-			if (dd) cbest = reduce_rows_key<KEY_NARROW, true>(sm.rows, R, t, mu, pbu, ul, 0u, best);
+			if (DEDUP && half) cbest = reduce_rows_key<KEY_NARROW, true, true>(sm.rows, R, t, mu, pbu, ul, 0u, best);
+			else if (dd) cbest = reduce_rows_key<KEY_NARROW, true>(sm.rows, R, t, mu, pbu, ul, 0u, best);
 			else cbest = reduce_rows_key<KEY_NARROW>(sm.rows, R, t, m, pbw, nullptr, 0u, best);
 		} else if constexpr (IsSymmetric<CD>::value) {
 			// saturated keys first; a block whose least sum reaches the cap
 			// scans again with exact 64-bit keys
 			const uint32_t cap = s2tc_scan_cap;
-			if (dd) cbest = reduce_rows_key<KEY_SAT, true>(sm.rows, R, t, mu, pbu, ul, cap, best);
+			if (DEDUP && half) cbest = reduce_rows_key<KEY_SAT, true, true>(sm.rows, R, t, mu, pbu, ul, cap, best);
+			else if (dd) cbest = reduce_rows_key<KEY_SAT, true>(sm.rows, R, t, mu, pbu, ul, cap, best);
 			else cbest = reduce_rows_key<KEY_SAT>(sm.rows, R, t, m, pbw, nullptr, cap, best);
 			if (best >= cap) {
 				if (dd) cbest = reduce_rows_key<KEY_WIDE, true>(sm.rows, R, t, mu, pbu, ul, 0u, best);
@@ -739,11 +814,11 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 		for (int p = 0; p < pbw; ++p) {
 			const int i = 16 * p + t;
 			const bool irow = i < m;
-			const int ai = irow ? (int)(sm.cand[i] >> 16) : 0;
+			const int ai = irow ? (int)((sm.cand[i] >> 16) & 255u) : 0;
 			int dv[16];
 #pragma unroll
 			for (int k = 0; k < 16; ++k) {
-				const int ak = (int)(sm.cand[k] >> 16);
+				const int ak = (int)((sm.cand[k] >> 16) & 255u);
 				const int f0 = adist(0, ak), f1 = adist(255, ak);
 				const int fk = f1 < f0 ? f1 : f0;
 				const int d = adist(ai, ak);
@@ -759,8 +834,8 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 		uint32_t best;
 		const uint32_t abest = reduce_rows_key<KEY_NARROW>(sm.rows, R, t, m, pbw, nullptr, 0u, best);
 		const int ai = min((int)(abest >> 16), m - 1), aj = min((int)(abest & 0xffffu), m - 1);
-		a0 = (int)(sm.cand[ai] >> 16);
-		a1 = (int)(sm.cand[aj] >> 16);
+		a0 = (int)((sm.cand[ai] >> 16) & 255u);
+		a1 = (int)((sm.cand[aj] >> 16) & 255u);
 	}
 	__syncthreads();
 

@@ -31,13 +31,12 @@ struct TileJobs {
 struct KernelTable {
 	const void *fast[3][2];       // [dxt][raw]: k_fast_edge (partial blocks), null for NORMALMAP
 	const void *fast_int[3][2][3];  // [dxt][raw][refine]: k_fast_interior (full blocks), null for NORMALMAP
-	const void *normal[2];        // [raw]: k_normal<CD, raw>
+	const void *normal[2][2];     // [many][raw]: k_normal<CD, raw, RB> (many: normal_many)
 	const void *normal_wide[2];   // [raw]: k_normal_wide<CD, raw> (group memory in global scratch)
 	int normal_smem_cand;         // LDS bytes per candidate slot of a 4-block workgroup (candidate words)
-	int normal_smem_row;          // LDS bytes per stored distance row of a 4-block workgroup
 	int normal_smem_fixed;        // plus these bytes (features of the 16 texel candidates of 4 blocks)
 	const void *fast_batch[3][3]; // [dxt][refine]: persistent quick-mode kernel over a job list
-	const void *normal_batch;     // persistent MODE_NORMAL kernel over a job list
+	const void *normal_batch[2];  // [many]: persistent MODE_NORMAL kernel over a job list
 	const void *normal_batch_wide;  // the same with group memory in global scratch
 	const void *all16[3][2];      // [dxt][raw]: MODE_NORMAL without random colours, one lane per block
 	const void *all16_batch[3][3];  // [dxt][refine]: its persistent batch form
@@ -48,17 +47,47 @@ struct KernelTable {
 };
 
 // Row blocks (16 rows each) of a block's distance matrix that the
-// random-candidate kernels keep in registers instead of LDS.
-#define S2TC_REG_RB 2
+// random-candidate kernels keep in registers instead of group memory.  The
+// kernels with two run four waves to a SIMD.  From five row blocks to eight
+// (49 to 112 random colours) group memory holds fewer workgroups than that, 11
+// to 6 to a CU, which the SIMDs share unevenly; with three row blocks in 168
+// registers twelve to 8 fit.  Measured (MI355X, 1024 x 1024, two -> three):
+// NORMALMAP 64 random colours 134.9 -> 117.4 us, 112 267 -> 235 us; SRGB 337 ->
+// 278 us and 1075 -> 975 us.  Outside that range, and where a launch has no
+// more workgroups than eight to a CU, the third row block only costs moves:
+// 48 random colours up to 8% slower, 128 SRGB 2%, 256 x 256 SRGB 8%.
+#define S2TC_RB_FEW 2
+#define S2TC_RB_MANY 3
+inline bool normal_many(int pbw, long long workgroups)
+{
+	return pbw >= 5 && pbw <= 8 && workgroups > 8 * 256;
+}
+
+#if defined(__HIP__) || defined(__HIPCC__)
+#define S2TC_HD __host__ __device__
+#else
+#define S2TC_HD
+#endif
+
+// Ints of row memory per block with pbw row blocks, rb of them in registers:
+// the other rows.  With three in registers and five in all, 560 instead of
+// 512, so that the tables of the scan over distinct colours hold a box of 160
+// cells (two ints a cell, three a candidate): 80 candidates fall on 63 of
+// them, a row block less, and twelve workgroups still fit a CU.
+S2TC_HD inline int normal_row_ints(int pbw, int rb)
+{
+	const int rows = 256 * (pbw > rb ? pbw - rb : 0);
+	return rb == S2TC_RB_MANY && rows < 560 ? 560 : rows;
+}
 
 // Group memory of a four-block workgroup of the random-candidate kernels
-// with pbw row blocks: 16 pbw candidate slots, the rows from 16 S2TC_REG_RB
-// on and the texel features.
-inline size_t normal_group_smem(const KernelTable &kt, int pbw)
+// with pbw row blocks: 16 pbw candidate slots, the row memory and the texel
+// features.
+inline size_t normal_group_smem(const KernelTable &kt, int pbw, bool many)
 {
-	const int stored = pbw > S2TC_REG_RB ? pbw - S2TC_REG_RB : 0;
-	return (size_t)kt.normal_smem_cand * 16 * (size_t)pbw + (size_t)kt.normal_smem_row * 16 * (size_t)stored +
-	       (size_t)kt.normal_smem_fixed;
+	const int rb = many ? S2TC_RB_MANY : S2TC_RB_FEW;
+	return (size_t)kt.normal_smem_cand * 16 * (size_t)pbw +
+	       (size_t)4 * sizeof(int) * (size_t)normal_row_ints(pbw, rb) + (size_t)kt.normal_smem_fixed;
 }
 
 extern "C" {

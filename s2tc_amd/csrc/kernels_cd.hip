@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(All16Waves<
 
 // MODE_NORMAL over one image: 16 lanes per block, 4 blocks per 64-lane
 // workgroup; tile `tile` covers raster blocks 4*tile .. 4*tile+3.
-template <int CD, bool RAW, bool DEDUP>
+template <int CD, bool RAW, int RB, bool DEDUP>
 S2TC_D void normal_image_tile(const uint32_t *__restrict__ src, int width, int height, uint8_t *__restrict__ dst,
                               int dxt, int nrandom, int refine, unsigned long long seed, int pbw,
                               unsigned block_base, const GroupSmem<CD> &sm, int tile, int g, int t)
@@ -223,25 +223,30 @@ S2TC_D void normal_image_tile(const uint32_t *__restrict__ src, int width, int h
 	}
 	const uint32_t bkey = s2tc_prng_block_key((uint64_t)seed, block_base + (uint32_t)b);
 	BlockOut o;
-	encode_block_normal<CD, DEDUP>(tex, t, w, h, dxt, nrandom, refine, bkey, pbw, sm, o);
+	encode_block_normal<CD, RB, DEDUP>(tex, t, w, h, dxt, nrandom, refine, bkey, pbw, sm, o);
 	if (have && t == 0) {
 		if (dxt == DXT1) store_block<DXT1>(dst, (size_t)b, o);
 		else store_block<DXT5>(dst, (size_t)b, o);
 	}
 }
 
+// Waves per SIMD the random-candidate kernels are compiled for: three with
+// three row blocks in registers (kernel_table.h says why), else four (left to
+// itself the compiler spares registers for a fifth: SRGB scans 4% slower).
+#define S2TC_RB_WAVES(RB) __attribute__((amdgpu_waves_per_eu(RB == S2TC_RB_MANY ? 3 : 4, RB == S2TC_RB_MANY ? 3 : 4)))
+
 // Candidates, rows and column features in LDS (nrandom <= S2TC_LDS_NRANDOM);
 // one workgroup per tile.
-template <int CD, bool RAW>
-__global__ __launch_bounds__(64) void k_normal(const uint32_t *__restrict__ src, int width, int height,
+template <int CD, bool RAW, int RB>
+__global__ __launch_bounds__(64) S2TC_RB_WAVES(RB) void k_normal(const uint32_t *__restrict__ src, int width, int height,
                                                uint8_t *__restrict__ dst, int dxt, int nrandom, int refine,
                                                unsigned long long seed, int pbw, unsigned block_base)
 {
 	extern __shared__ __align__(16) uint8_t smem[];
 	const int lane = (int)threadIdx.x;
 	const int g = lane >> 4, t = lane & 15;
-	const GroupSmem<CD> sm = group_smem<CD>(smem, g, 16 * pbw);
-	normal_image_tile<CD, RAW, true>(src, width, height, dst, dxt, nrandom, refine, seed, pbw, block_base, sm,
+	const GroupSmem<CD> sm = group_smem<CD, RB>(smem, g, 16 * pbw);
+	normal_image_tile<CD, RAW, RB, true>(src, width, height, dst, dxt, nrandom, refine, seed, pbw, block_base, sm,
 	                                 xcd_local_id((int)blockIdx.x, (int)gridDim.x), g, t);
 }
 
@@ -258,12 +263,12 @@ __global__ __launch_bounds__(64) void k_normal_wide(const uint32_t *__restrict__
 {
 	const int lane = (int)threadIdx.x;
 	const int g = lane >> 4, t = lane & 15;
-	const size_t wg_bytes = 4 * group_smem_bytes<CD>(16 * pbw);
-	const GroupSmem<CD> sm = group_smem<CD>(gmem + (size_t)blockIdx.x * wg_bytes, g, 16 * pbw);
+	const size_t wg_bytes = 4 * group_smem_bytes<CD, S2TC_RB_FEW>(16 * pbw);
+	const GroupSmem<CD> sm = group_smem<CD, S2TC_RB_FEW>(gmem + (size_t)blockIdx.x * wg_bytes, g, 16 * pbw);
 	const int bw = (width + 3) >> 2, bh = (height + 3) >> 2;
 	const int ntiles = (bw * bh + 3) >> 2;
 	for (int tile = xcd_local_id((int)blockIdx.x, (int)gridDim.x); tile < ntiles; tile += (int)gridDim.x) {
-		normal_image_tile<CD, RAW, false>(src, width, height, dst, dxt, nrandom, refine, seed, pbw, block_base, sm,
+		normal_image_tile<CD, RAW, S2TC_RB_FEW, false>(src, width, height, dst, dxt, nrandom, refine, seed, pbw, block_base, sm,
 		                                  tile, g, t);
 		__syncthreads();
 	}
@@ -384,7 +389,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 	all16_batch_tiles<CD, DXT, REFINE>(jobs, tile_jobs, nblocks, ntiles);
 }
 
-template <int CD, bool DEDUP>
+template <int CD, int RB, bool DEDUP>
 S2TC_D void normal_batch_tile(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
                               long long nblocks, const GroupSmem<CD> &sm, int tile, int g, int t)
 {
@@ -407,7 +412,7 @@ S2TC_D void normal_batch_tile(const JobDesc *__restrict__ jobs, const TileJobs *
 	const uint32_t bkey = s2tc_prng_block_key((uint64_t)j.seed, (uint32_t)b);
 	const int pbw = (16 + (j.nrandom > 0 ? j.nrandom : 0) + 15) / 16;
 	BlockOut o;
-	encode_block_normal<CD, DEDUP>(tex, t, w, h, j.dxt, j.nrandom, j.refine, bkey, pbw, sm, o);
+	encode_block_normal<CD, RB, DEDUP>(tex, t, w, h, j.dxt, j.nrandom, j.refine, bkey, pbw, sm, o);
 	if (have && t == 0) {
 		if (j.dxt == DXT1) store_block<DXT1>(j.dst, (size_t)b, o);
 		else store_block<DXT5>(j.dst, (size_t)b, o);
@@ -450,14 +455,14 @@ S2TC_D BlockIn fetch_block(const JobDesc *__restrict__ jobs, TileJobs tj, int ti
 	return in;
 }
 
-template <int CD> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<CD> &sm, int t)
+template <int CD, int RB> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<CD> &sm, int t)
 {
 	const int x = t >> 2, y = t & 3;
 	uint32_t tex = 0;
 	if (x < in.w && y < in.h) tex = in.raw ? quant_none_rt(in.tex, in.dxt) : in.tex;
 	const int pbw = (16 + (in.nrandom > 0 ? in.nrandom : 0) + 15) / 16;
 	BlockOut o;
-	encode_block_normal<CD, true>(tex, t, in.w, in.h, in.dxt, in.nrandom, in.refine, in.bkey, pbw, sm, o);
+	encode_block_normal<CD, RB, true>(tex, t, in.w, in.h, in.dxt, in.nrandom, in.refine, in.bkey, pbw, sm, o);
 	if (in.have && t == 0) {
 		if (in.dxt == DXT1) store_block<DXT1>(in.dst, (size_t)in.b, o);
 		else store_block<DXT5>(in.dst, (size_t)in.b, o);
@@ -468,14 +473,14 @@ template <int CD> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<
 // job and texels of tile T + G are in flight and the tile record of T + 2G
 // (G = grid size; indices past the end are clamped to the last tile, whose
 // inputs are then fetched and never used).
-template <int CD>
-__global__ __launch_bounds__(64) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
+template <int CD, int RB>
+__global__ __launch_bounds__(64) S2TC_RB_WAVES(RB) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
                                                      long long nblocks, int ntiles, int pbw_max)
 {
 	extern __shared__ __align__(16) uint8_t smem[];
 	const int lane = (int)threadIdx.x;
 	const int g = lane >> 4, t = lane & 15;
-	const GroupSmem<CD> sm = group_smem<CD>(smem, g, 16 * pbw_max);
+	const GroupSmem<CD> sm = group_smem<CD, RB>(smem, g, 16 * pbw_max);
 	const int G = (int)gridDim.x;
 	int tile = xcd_local_id((int)blockIdx.x, G);
 	if (tile >= ntiles) return;
@@ -489,7 +494,7 @@ __global__ __launch_bounds__(64) void k_normal_batch(const JobDesc *__restrict__
 	for (; tile < ntiles; tile += G) {
 		const BlockIn nxt = fetch_block(jobs, tjn, min(tile + G, ntiles - 1), nblocks, g, t);
 		tjn = tile_at(tile + 2 * G);
-		encode_fetched<CD>(cur, sm, t);
+		encode_fetched<CD, RB>(cur, sm, t);
 		__syncthreads();
 		cur = nxt;
 	}
@@ -504,10 +509,10 @@ __global__ __launch_bounds__(64) void k_normal_batch_wide(const JobDesc *__restr
 {
 	const int lane = (int)threadIdx.x;
 	const int g = lane >> 4, t = lane & 15;
-	const size_t wg_bytes = 4 * group_smem_bytes<CD>(16 * pbw_max);
-	const GroupSmem<CD> sm = group_smem<CD>(gmem + (size_t)blockIdx.x * wg_bytes, g, 16 * pbw_max);
+	const size_t wg_bytes = 4 * group_smem_bytes<CD, S2TC_RB_FEW>(16 * pbw_max);
+	const GroupSmem<CD> sm = group_smem<CD, S2TC_RB_FEW>(gmem + (size_t)blockIdx.x * wg_bytes, g, 16 * pbw_max);
 	for (int tile = xcd_local_id((int)blockIdx.x, (int)gridDim.x); tile < ntiles; tile += (int)gridDim.x) {
-		normal_batch_tile<CD, false>(jobs, tile_jobs, nblocks, sm, tile, g, t);
+		normal_batch_tile<CD, S2TC_RB_FEW, false>(jobs, tile_jobs, nblocks, sm, tile, g, t);
 		__syncthreads();
 	}
 }
@@ -635,7 +640,8 @@ extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 #else
 	for (int d = 0; d < 3; ++d) kt->fast_batch[d][0] = kt->fast_batch[d][1] = kt->fast_batch[d][2] = nullptr;
 #endif
-	kt->normal_batch = (const void *)k_normal_batch<S2TC_CD>;
+	kt->normal_batch[0] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_FEW>;
+	kt->normal_batch[1] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_MANY>;
 	kt->normal_batch_wide = (const void *)k_normal_batch_wide<S2TC_CD>;
 	kt->error[DXT1][0] = (const void *)k_colordist_error<S2TC_CD, DXT1, false>;
 	kt->error[DXT3][0] = (const void *)k_colordist_error<S2TC_CD, DXT3, false>;
@@ -665,8 +671,10 @@ extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 #undef S2TC_AL3
 	}
 #undef S2TC_AB3
-	kt->normal[0] = (const void *)k_normal<S2TC_CD, false>;
-	kt->normal[1] = (const void *)k_normal<S2TC_CD, true>;
+	kt->normal[0][0] = (const void *)k_normal<S2TC_CD, false, S2TC_RB_FEW>;
+	kt->normal[0][1] = (const void *)k_normal<S2TC_CD, true, S2TC_RB_FEW>;
+	kt->normal[1][0] = (const void *)k_normal<S2TC_CD, false, S2TC_RB_MANY>;
+	kt->normal[1][1] = (const void *)k_normal<S2TC_CD, true, S2TC_RB_MANY>;
 	kt->normal_wide[0] = (const void *)k_normal_wide<S2TC_CD, false>;
 	kt->normal_wide[1] = (const void *)k_normal_wide<S2TC_CD, true>;
 #if defined(S2TC_NM_TABLE) || defined(S2TC_SRGB_Y_TABLE)
@@ -676,6 +684,5 @@ extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 #endif
 	kt->set_scan_cap = (const void *)k_set_scan_cap<S2TC_CD>;
 	kt->normal_smem_cand = (int)(4 * sizeof(uint32_t));
-	kt->normal_smem_row = (int)(4 * S2TC_RS * sizeof(int));
 	kt->normal_smem_fixed = (int)(4 * 16 * sizeof(Dist<S2TC_CD>::F));
 }

@@ -107,13 +107,14 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 	}
 	for (auto &c : classes) {
 		const KernelTable &kt = kernel_table(c.cd);
+		c.ntiles = (int)((c.nblocks + c.tile - 1) / c.tile);
+		const bool many = normal_many(c.pbw_max, c.ntiles);
 		c.kernel = c.wide     ? kt.normal_batch_wide
-		           : c.normal ? kt.normal_batch
+		           : c.normal ? kt.normal_batch[many]
 		           : c.all16  ? kt.all16_batch[c.dxt][c.refine]
 		                      : kt.fast_batch[c.dxt][c.refine];
 		if (!c.kernel) return set_error(S2TC_E_ARG, "no batch kernel for distance %d", c.cd);
-		c.ntiles = (int)((c.nblocks + c.tile - 1) / c.tile);
-		c.smem = c.normal && !c.wide ? normal_group_smem(kt, c.pbw_max) : 0;
+		c.smem = c.normal && !c.wide ? normal_group_smem(kt, c.pbw_max, many) : 0;
 		if (c.wide) wide_launch_shape(kt, c.pbw_max, c.ntiles, device_cu_count(), c.wide_grid, c.scratch);
 		tile_ranges(c.jobs, c.nblocks, c.tile, c.ntiles, c.tiles);
 		if (c.all16) {
@@ -122,9 +123,9 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 			c.forms[FORM_LANE_2WAVES] = k2 != c.kernel ? k2 : nullptr;
 			if (with_forms) {
 				// the random-candidate kernel runs nrandom-0 jobs as they are
-				c.forms[FORM_ROW16] = kt.normal_batch;
+				c.forms[FORM_ROW16] = kt.normal_batch[0];
 				c.ntiles4 = (int)((c.nblocks + 3) / 4);
-				c.smem4 = normal_group_smem(kt, 1);
+				c.smem4 = normal_group_smem(kt, 1, false);
 				tile_ranges(c.jobs, c.nblocks, 4, c.ntiles4, c.tiles4);
 			}
 		}
@@ -183,7 +184,7 @@ void plan_set_scratch(std::vector<ClassPlan> &classes, uint8_t *dev)
 
 void wide_launch_shape(const KernelTable &kt, int pbw, long long ntiles, int ncu, int &grid, size_t &bytes)
 {
-	const size_t wg = normal_group_smem(kt, pbw);
+	const size_t wg = normal_group_smem(kt, pbw, false);
 	const long long cap = std::max(1LL, (long long)(((size_t)1 << 30) / wg));
 	grid = (int)std::max(1LL, std::min(ntiles, std::min(4LL * ncu, cap)));
 	bytes = wg * (size_t)grid;

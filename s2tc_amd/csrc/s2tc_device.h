@@ -329,8 +329,15 @@ struct Recip {
 	}
 	S2TC_D uint32_t div(uint32_t x) const { return ((x & 0x1fffu) * m) >> 18; }
 };
-// ((S << 1) + n) / (n << 1): round-half-up mean (:547-549); s <= 255 n, n <= 16
-S2TC_D int rmean(int s, int n) { return (int)Recip((uint32_t)(n << 1)).div((uint32_t)((s << 1) + n)); }
+// ((S << 1) + n) / (n << 1): round-half-up mean (:547-549) for 0 <= S <= 255 n
+// and 1 <= n <= 16, as trunc(S / n + 1/2 + 1/64): the quotients are multiples
+// of 1 / 2n >= 1/32, so the extra 1/64 never reaches the next integer, and it
+// outweighs the error of the approximate reciprocal (below 2^-13).
+struct Mean {
+	float rn;
+	S2TC_D explicit Mean(int n) : rn(__builtin_amdgcn_rcpf((float)n)) {}
+	S2TC_D uint32_t of(uint32_t s) const { return (uint32_t)__builtin_fmaf((float)s, rn, 0.515625f); }
+};
 
 // 2-bit colour index word fix-ups (:802-804, :810-812)
 S2TC_D uint32_t keep_ones(uint32_t bits)

@@ -155,11 +155,12 @@ int launch_encode(const EncodeArgs &a, hipStream_t stream, void *ext_scratch, si
 	unsigned long long seed = a.seed;
 	unsigned block_base = a.block_index_base;
 	if (nrandom <= S2TC_LDS_NRANDOM) {
-		size_t smem = normal_group_smem(kt, pbw);
+		dim3 grid((unsigned)((nb + 3) / 4)), block(64);
+		const bool many = normal_many(pbw, grid.x);
+		size_t smem = normal_group_smem(kt, pbw, many);
 		void *args[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&dxt,
 		                (void *)&nrandom, (void *)&refine, (void *)&seed, (void *)&pbw, (void *)&block_base};
-		dim3 grid((unsigned)((nb + 3) / 4)), block(64);
-		return hip_check(hipLaunchKernel(kt.normal[raw], grid, block, args, smem, stream), "launch k_normal");
+		return hip_check(hipLaunchKernel(kt.normal[many][raw], grid, block, args, smem, stream), "launch k_normal");
 	}
 	// more candidates than LDS holds: group memory in the caller's scratch, or
 	// in stream-ordered scratch that lives exactly as long as this launch
