@@ -43,6 +43,10 @@ int normal_pbw(int nrandom);
 // around the launch.
 int launch_encode(const EncodeArgs &a, hipStream_t stream, void *ext_scratch = nullptr, size_t ext_bytes = 0);
 
+// Upload from pinned host memory by its device address (util.hip): n bytes
+// rounded up to 16, which both buffers hold, at 16-byte aligned addresses.
+int launch_pull(void *dst, const void *src, size_t n, hipStream_t st);
+
 // rgb565_image on the device (dither.hip); d_scratch holds
 // rgb565_scratch_bytes(w, h, dither).
 // d_carry_in / d_carry_out (4 bytes each, apart; SIMPLE only): the image is a

@@ -3,8 +3,8 @@
 // tx_compress_dxtn follows s2tc_libtxc_dxtn.cpp:142-299: environment
 // configuration read on every call, GL format switch, rgb565_image, the
 // raster block loop and the destination row padding rule.  The quantization
-// and the block loop run on the GPU; the host uploads the source, downloads
-// the blocks and lays out the destination rows.  Each call borrows a
+// and the block loop run on the GPU; the host copies the source into pinned
+// memory and lays out the destination rows from the blocks.  Each call borrows a
 // context (stream + device buffers) from a pool, so concurrent callers on
 // different threads do not share buffers.
 #include "s2tc_internal.h"
@@ -43,10 +43,11 @@ struct DevBuf {
 	}
 };
 
-// Pinned host memory (hipHostMalloc): DMA-able staging for the host-buffer
-// entry points, grown on demand and kept with the context.
+// Pinned host memory (hipHostMalloc): staging for the host-buffer entry
+// points that copies and kernels (at `dev`) reach, grown on demand and kept
+// with the context.
 struct HostBuf {
-	void *p = nullptr;
+	void *p = nullptr, *dev = nullptr;
 	size_t cap = 0;
 	int ensure(size_t n)
 	{
@@ -55,101 +56,126 @@ struct HostBuf {
 		p = nullptr;
 		cap = 0;
 		n = (n + 4095) & ~(size_t)4095;
-		if (int r = hip_check(hipHostMalloc(&p, n, hipHostMallocDefault), "hipHostMalloc")) return r;
+		if (int r = hip_check(hipHostMalloc(&p, n, hipHostMallocMapped), "hipHostMalloc")) return r;
+		if (int r = hip_check(hipHostGetDevicePointer(&dev, p, 0), "hipHostGetDevicePointer")) {
+			(void)hipHostFree(p);
+			p = nullptr;
+			return r;
+		}
 		cap = n;
 		return 0;
 	}
 	uint8_t *data() const { return (uint8_t *)p; }
 };
 
-// Inputs up to this size are copied into pinned staging before the upload;
-// larger ones stream through two pinned buffers of this size.
-static const size_t kStageMax = 8u << 20;
-// Host threads (the caller's included) that fill a staging buffer.
-static const unsigned kUploadThreads = 4;
+// How a call's host data reaches the kernels and comes back, by size; measured
+// (MI355X, whole calls, against a copy into staging, a DMA, the kernels, a DMA
+// back and the rows laid out, one after the other):
+//   up to kDirectMax, the kernels read the pinned copy of the source, and write
+//   blocks of up to kDirectMax to pinned memory: 256 x 256 RGBA quick 36 -> 21
+//   us, with the SIMPLE dither 50 -> 41 us (two passes over the bus still beat
+//   a DMA at 512 KiB, and lose at 1 MiB);
+//   up to kBandMin, the upload kernel runs over each half while the other is
+//   copied: 1024 x 1024 SIMPLE 216 -> 175 us (four pieces: the same);
+//   above, in bands (encode_host_bands) with uploads of kChunk through a ring of
+//   kRing pinned buffers: 2048 x 2048 NONE 601 -> 483 us, 4096 x 4096 DXT5
+//   SIMPLE 2.04 -> 1.86 ms (2 MiB: 1.93 ms; 512 KiB: 1.99 ms).  In bands from 4
+//   MiB on, 1024 x 1024 SIMPLE took 253 us: starting the threads and the
+//   smaller launches cost more than the overlap gives.
+static const size_t kDirectMax = 512u << 10;
+static const size_t kBandMin = 8u << 20;
+static const size_t kChunk = 1u << 20, kRing = 12;
+// Host threads (the caller's included) that copy; three to six measure alike,
+// eight are 5% slower.
+static const unsigned kCopyThreads = 4;
+// Bands whose blocks may be on their way back.
+static const int kOutRing = 4;
+
+static unsigned copy_helpers()
+{
+	const unsigned hw = std::thread::hardware_concurrency();
+	return std::max(1u, std::min(kCopyThreads, hw ? hw : 1u)) - 1;
+}
 
 struct Ctx {
 	hipStream_t stream = nullptr;
-	hipStream_t copy_stream = nullptr;    // uploads of a call encoded in bands (created on first use)
-	hipStream_t dither_stream = nullptr;  // its per-band quantization
-	hipStream_t d2h_stream = nullptr;     // and the download of each encoded band
+	hipStream_t copy_stream[2] = {};    // uploads of a call encoded in bands (created on first use)
 	DevBuf src, q, out, scratch;
-	HostBuf in_stage, in_stage2, host_out;
-	hipEvent_t stage_ev[2] = {nullptr, nullptr};  // last DMA out of in_stage / in_stage2
-	hipEvent_t band_ev = nullptr;                 // uploaded rows handed to the dither / compute stream
-	hipEvent_t dither_ev = nullptr;               // a quantized band handed to the compute stream
-	hipEvent_t enc_ev = nullptr;                  // an encoded band handed to the download stream
+	HostBuf in_stage, host_out;
+	hipEvent_t stage_ev[kRing] = {};    // last upload out of each buffer of in_stage
+	hipEvent_t out_ev[kOutRing] = {};   // encoded bands
 	// per-block calls: one mapped pinned page that the kernel reads the block's
 	// texels from (offset 0) and writes its encoding to (offset 64)
 	uint8_t *blk_host = nullptr;
 	void *blk_dev = nullptr;
 };
 
-// A large upload in chunks of kStageMax bytes through the two pinned
-// buffers: while the DMA of chunk i runs, the host threads copy chunk i + 1
-// into the other buffer (one host thread alone copies pageable memory well
-// below the link rate).  A buffer is refilled only after the event of the
-// DMA that last read it.  The DMAs go to `st`; after each one is queued,
-// on_chunk (if given) learns how many leading bytes are then on their way.
-static int upload_large(Ctx *c, void *dst, const void *src, size_t n, hipStream_t st,
-                        const std::function<int(size_t)> &on_chunk = nullptr)
+// Whether the work that an event follows is done (a query that is not leaves no
+// error behind for the next launch to find).
+static bool event_done(hipEvent_t ev)
 {
-	int rc = c->in_stage.ensure(kStageMax);
-	if (!rc) rc = c->in_stage2.ensure(kStageMax);
-	for (int b = 0; b < 2 && !rc; ++b)
-		if (!c->stage_ev[b])
-			rc = hip_check(hipEventCreateWithFlags(&c->stage_ev[b], hipEventDisableTiming), "hipEventCreate");
-	if (rc) return rc;
-	const long nchunks = (long)((n + kStageMax - 1) / kStageMax);
-	const unsigned hw = std::thread::hardware_concurrency();
-	const unsigned nt = std::max(1u, std::min(kUploadThreads, hw ? hw : 1u));
-	std::unique_ptr<std::atomic<unsigned>[]> done(new std::atomic<unsigned>[(size_t)nchunks]);
-	for (long i = 0; i < nchunks; ++i) done[i].store(0);
-	std::atomic<long> open{-1};  // the highest chunk the threads may copy
-	std::atomic<bool> abort{false};
-	uint8_t *bufs[2] = {c->in_stage.data(), c->in_stage2.data()};
-	auto copy_slice = [&](long i, unsigned t) {
-		const size_t off = (size_t)i * kStageMax, len = std::min(kStageMax, n - off);
-		size_t lo, hi;
-		stage_slice(len, nt, t, lo, hi);
-		if (hi > lo) memcpy(bufs[i & 1] + lo, (const uint8_t *)src + off + lo, hi - lo);
-		done[i].fetch_add(1, std::memory_order_release);
-	};
-	std::vector<std::thread> workers;
-	for (unsigned t = 1; t < nt; ++t)
-		workers.emplace_back([&, t] {
-			for (long i = 0; i < nchunks; ++i) {
-				while (open.load(std::memory_order_acquire) < i) {
-					if (abort.load(std::memory_order_acquire)) return;
-					std::this_thread::yield();
-				}
-				if (abort.load(std::memory_order_acquire)) return;
-				copy_slice(i, t);
+	if (hipEventQuery(ev) == hipSuccess) return true;
+	(void)hipGetLastError();
+	return false;
+}
+
+// Upload of a source in chunks through the ring of pinned buffers: while the
+// upload kernel of a chunk runs, the host threads copy the next ones (one host
+// thread alone copies pageable memory well below the link rate).  A buffer is
+// refilled only after the event of the upload that last read it; a call leaves
+// none behind, so the buffers start out free.  Chunks alternate between st0 and
+// st1: two streams hide the gap between one stream's kernels.  on_chunk (if
+// given) learns of every queued chunk and how many leading bytes are then on
+// their way, after the next chunk is queued.
+static int upload_chunks(Ctx *c, CopyCrew &crew, void *dst, hipStream_t st0, hipStream_t st1,
+                         const std::function<int(size_t, size_t)> &on_chunk = nullptr)
+{
+	for (auto &ev : c->stage_ev)
+		if (!ev)
+			if (int r = hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return r;
+	size_t open = std::min(crew.nchunks, crew.ring);
+	crew.open_chunks(open);
+	for (size_t i = 0; i < crew.nchunks; ++i) {
+		while (!crew.chunk_copied(i))
+			if (!crew.step()) std::this_thread::yield();
+		const size_t off = i * crew.chunk, len = crew.chunk_len(i);
+		const hipStream_t st = i & 1 ? st1 : st0;
+		if (int r = launch_pull((uint8_t *)dst + off, (uint8_t *)c->in_stage.dev + crew.ring_offset(i), len, st))
+			return r;
+		if (on_chunk || crew.nchunks > crew.ring)
+			if (int r = hip_check(hipEventRecord(c->stage_ev[i % crew.ring], st), "hipEventRecord")) return r;
+		// what the previous chunk completed, while this one is on its way
+		if (on_chunk && i)
+			if (int r = on_chunk(i - 1, off)) return r;
+		// open the buffers whose upload ended; the next chunk's by waiting
+		while (open < crew.nchunks && open <= i + crew.ring) {
+			hipEvent_t ev = c->stage_ev[open % crew.ring];
+			if (open == i + 1) {
+				if (int r = hip_check(hipEventSynchronize(ev), "hipEventSynchronize")) return r;
+			} else if (!event_done(ev)) {
+				break;
 			}
-		});
-	for (long i = 0; i < nchunks && !rc; ++i) {
-		rc = hip_check(hipEventSynchronize(c->stage_ev[i & 1]), "hipEventSynchronize");
-		if (rc) break;
-		open.store(i, std::memory_order_release);
-		copy_slice(i, 0);
-		while (done[i].load(std::memory_order_acquire) < nt) std::this_thread::yield();
-		const size_t off = (size_t)i * kStageMax, len = std::min(kStageMax, n - off);
-		rc = hip_check(hipMemcpyAsync((uint8_t *)dst + off, bufs[i & 1], len, hipMemcpyHostToDevice, st), "H2D");
-		if (!rc) rc = hip_check(hipEventRecord(c->stage_ev[i & 1], st), "hipEventRecord");
-		if (!rc && on_chunk) rc = on_chunk(off + len);
+			crew.open_chunks(++open);
+		}
 	}
-	if (rc) abort.store(true, std::memory_order_release);
-	for (auto &w : workers) w.join();
-	return rc;
+	return on_chunk ? on_chunk(crew.nchunks - 1, crew.n) : 0;
 }
 
 // host -> device upload of a caller's buffer on the context's stream
 static int upload(Ctx *c, void *dst, const void *src, size_t n)
 {
-	if (n > kStageMax) return upload_large(c, dst, src, n, c->stream);
-	if (int r = c->in_stage.ensure(n)) return r;
-	memcpy(c->in_stage.p, src, n);
-	return hip_check(hipMemcpyAsync(dst, c->in_stage.p, n, hipMemcpyHostToDevice, c->stream), "H2D");
+	if (n <= 2 * kDirectMax) {
+		if (int r = c->in_stage.ensure(n)) return r;
+		memcpy(c->in_stage.p, src, n);
+		return launch_pull(dst, c->in_stage.dev, n, c->stream);
+	}
+	// halves, or pieces of 4 MiB by several threads
+	const size_t chunk = std::min(((n + 1) / 2 + 4095) & ~(size_t)4095, (size_t)4 << 20);
+	const size_t ring = std::min((size_t)4, (n + chunk - 1) / chunk);
+	if (int r = c->in_stage.ensure(ring * chunk)) return r;
+	CopyCrew crew((const uint8_t *)src, n, c->in_stage.data(), chunk, ring);
+	if (n > 2 * chunk) crew.start(copy_helpers());
+	return upload_chunks(c, crew, dst, c->stream, c->stream);
 }
 
 static std::mutex g_pool_mu;
@@ -225,135 +251,159 @@ static EnvConfig read_env()
 // Rows per band of a large call (a multiple of 4: whole block rows): the
 // upload of later rows overlaps the dither and encode of earlier ones.  At
 // least 512 rows, and at least 2^18 blocks per band, which the one-lane-per-
-// block encoders need to fill the GPU (measured: 8192-wide normal map best at
-// 512 rows, 4096-wide tiles at 1024).
-static int band_rows(int width)
+// block encoders need to fill the GPU (8192 x 4096 with 2^17: 2.6 instead of
+// 2.4 ms), or half the image.
+static int band_rows(int width, int height)
 {
-	const long long r = ((1LL << 22) + width - 1) / width;
-	return (int)std::max(512LL, (r + 3) & ~3LL);
+	const long long r = std::max(512LL, ((1LL << 22) + width - 1) / width);
+	return (int)((std::min(r, (height + 1LL) / 2) + 3) & ~3LL);
 }
 
-// Large sources (more than one staging chunk, more than one band) with the
-// NONE or SIMPLE dither: the uploads run on the copy stream, and each band of
-// band_rows(width) rows is quantized on the dither stream and encoded on the
-// compute stream as soon as its rows are uploaded (the SIMPLE scan of a band uses few
-// CUs for a serial walk, so it runs beside the previous band's encode); each
-// band's blocks download on a fourth stream, beside the later uploads.
-// SIMPLE carries its error state from band to band on the device; the encoder
-// numbers the blocks of a band from the band's first block, so the random
-// candidates are those of the whole image.
+// Large sources (above kBandMin) with the NONE or SIMPLE dither: the uploads
+// run on the copy streams, and each band of rows is quantized and encoded on the
+// compute stream as soon as its rows are uploaded, beside the later uploads (a
+// band computes in less time than it uploads).  SIMPLE carries its error state
+// from band to band on the device; the encoder numbers the blocks of a band from
+// the band's first block, so the random candidates are those of the whole image,
+// and writes them to pinned memory itself.  No stream for each kind of work: the
+// hardware queues of a process are few, and streams that share one wait for each
+// other.  The rows of finished bands go to rows_dest (if given) while later ones
+// are on their way.
 static int encode_host_bands(Ctx *c, int srccomps, int width, int height, const uint8_t *src, int dxt,
-                             const EncodeArgs &base, int dither, int alphabits)
+                             const EncodeArgs &base, int dither, int alphabits, uint8_t *rows_dest, size_t row_pitch)
 {
-	const int brows = band_rows(width);
+	const int brows = band_rows(width, height);
 	const size_t row_bytes = (size_t)width * srccomps;
 	const size_t n = (size_t)width * height;
 	const int bw = (width + 3) / 4, bb = block_bytes(dxt);
-	const int nbands = (height + brows - 1) / brows;
+	// the last rows in bands of half the size: what is left to do after the last
+	// upload is short
+	const int full = (height - 1) / brows * brows, half = std::max(4, brows / 2 & ~3);
+	const int nbands = full / brows + (height - full + half - 1) / half;
+	const auto band_row = [&](int b) {
+		return (long long)b * brows <= full ? b * brows
+		                                    : (int)std::min((long long)height, full + (b - full / brows) * (long long)half);
+	};
 	const bool fused = dither == DITHER_NONE && srccomps == 4;
+	size_t scratch = 0;
+	for (int b = 0; b < nbands; ++b)
+		scratch = std::max(scratch, rgb565_scratch_bytes(width, band_row(b + 1) - band_row(b), dither));
 	if (!fused) {
 		if (int r = c->q.ensure(n * 4)) return r;
-		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, brows, dither) + 256)) return r;
+		if (int r = c->scratch.ensure(scratch + 256)) return r;
 	}
-	if (!c->copy_stream)
-		if (int r = hip_check(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking), "hipStreamCreate"))
-			return r;
-	if (!c->dither_stream)
-		if (int r = hip_check(hipStreamCreateWithFlags(&c->dither_stream, hipStreamNonBlocking), "hipStreamCreate"))
-			return r;
-	if (!c->d2h_stream)
-		if (int r = hip_check(hipStreamCreateWithFlags(&c->d2h_stream, hipStreamNonBlocking), "hipStreamCreate"))
-			return r;
-	if (!c->enc_ev)
-		if (int r = hip_check(hipEventCreateWithFlags(&c->enc_ev, hipEventDisableTiming), "hipEventCreate"))
-			return r;
-	const size_t obytes = (size_t)bw * ((height + 3) / 4) * bb;
-	if (int r = c->host_out.ensure(obytes)) return r;
-	if (!c->band_ev)
-		if (int r = hip_check(hipEventCreateWithFlags(&c->band_ev, hipEventDisableTiming), "hipEventCreate"))
-			return r;
-	if (!c->dither_ev)
-		if (int r = hip_check(hipEventCreateWithFlags(&c->dither_ev, hipEventDisableTiming), "hipEventCreate"))
-			return r;
-	uint8_t *carry = (uint8_t *)c->scratch.p + rgb565_scratch_bytes(width, brows, dither);
-	int next = 0;
-	auto on_chunk = [&](size_t uploaded) -> int {
+	for (auto &st : c->copy_stream)
+		if (!st)
+			if (int r = hip_check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate")) return r;
+	for (auto &ev : c->out_ev)
+		if (!ev)
+			if (int r = hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return r;
+	if (int r = c->in_stage.ensure(kRing * kChunk)) return r;
+	CopyCrew crew(src, n * srccomps, c->in_stage.data(), kChunk, kRing);
+	if (rows_dest) crew.set_rows(rows_dest, c->host_out.data(), (size_t)bw * bb, row_pitch, (height + 3) / 4);
+	crew.start(copy_helpers());
+	uint8_t *carry = (uint8_t *)c->scratch.p + scratch;
+	int next = 0, back = 0;  // bands launched, bands whose blocks have come back
+	// opens the rows of the bands that came back; waits for those before `until`
+	auto collect = [&](int until) -> int {
+		while (back < next) {
+			hipEvent_t ev = c->out_ev[back % kOutRing];
+			if (back < until) {
+				if (int r = hip_check(hipEventSynchronize(ev), "hipEventSynchronize")) return r;
+			} else if (!event_done(ev)) {
+				break;
+			}
+			++back;
+			crew.open_rows((band_row(back) + 3) / 4);
+		}
+		return 0;
+	};
+	auto on_chunk = [&](size_t chunk, size_t uploaded) -> int {
 		bool waited = false;
-		while (next < nbands && (size_t)std::min(height, (next + 1) * brows) * row_bytes <= uploaded) {
-			hipStream_t first = fused ? c->stream : c->dither_stream;  // the band's first user
+		if (int r = collect(0)) return r;
+		while (next < nbands && (size_t)band_row(next + 1) * row_bytes <= uploaded) {
 			if (!waited) {
-				if (int r = hip_check(hipEventRecord(c->band_ev, c->copy_stream), "hipEventRecord")) return r;
-				if (int r = hip_check(hipStreamWaitEvent(first, c->band_ev, 0), "hipStreamWaitEvent")) return r;
+				// the last chunk of either copy stream
+				for (size_t i = chunk ? chunk - 1 : 0; i <= chunk; ++i)
+					if (int r = hip_check(hipStreamWaitEvent(c->stream, c->stage_ev[i % crew.ring], 0),
+					                      "hipStreamWaitEvent"))
+						return r;
 				waited = true;
 			}
-			const int r0 = next * brows, rows = std::min(brows, height - r0);
+			const int r0 = band_row(next), rows = band_row(next + 1) - r0;
 			const uint8_t *bsrc = (const uint8_t *)c->src.p + (size_t)r0 * row_bytes;
 			EncodeArgs a = base;
 			a.height = rows;
 			a.block_index_base = (uint32_t)((size_t)(r0 / 4) * bw);
-			a.dst = (uint8_t *)c->out.p + (size_t)(r0 / 4) * bw * bb;
 			if (fused) {
 				a.src = bsrc;
 				a.src_kind = S2TC_SRC_RGBA8;
 			} else {
 				uint8_t *bq = (uint8_t *)c->q.p + (size_t)r0 * width * 4;
-				if (int r = launch_rgb565(bsrc, srccomps, width, rows, alphabits, dither, bq, c->scratch.p,
-				                          c->dither_stream, next > 0 ? carry + 4 * (next & 1) : nullptr,
-				                          carry + 4 * ((next + 1) & 1)))
+				if (int r = launch_rgb565(bsrc, srccomps, width, rows, alphabits, dither, bq, c->scratch.p, c->stream,
+				                          next > 0 ? carry + 4 * (next & 1) : nullptr, carry + 4 * ((next + 1) & 1)))
 					return r;
-				if (int r = hip_check(hipEventRecord(c->dither_ev, c->dither_stream), "hipEventRecord")) return r;
-				if (int r = hip_check(hipStreamWaitEvent(c->stream, c->dither_ev, 0), "hipStreamWaitEvent")) return r;
 				a.src = bq;
 				a.src_kind = S2TC_SRC_QUANTIZED;
 			}
+			a.dst = (uint8_t *)c->host_out.dev + (size_t)(r0 / 4) * bw * bb;
 			if (int r = launch_encode(a, c->stream)) return r;
-			const size_t o0 = (size_t)(r0 / 4) * bw * bb, o1 = std::min(obytes, (size_t)((r0 + rows + 3) / 4) * bw * bb);
-			if (int r = hip_check(hipEventRecord(c->enc_ev, c->stream), "hipEventRecord")) return r;
-			if (int r = hip_check(hipStreamWaitEvent(c->d2h_stream, c->enc_ev, 0), "hipStreamWaitEvent")) return r;
-			if (int r = hip_check(hipMemcpyAsync(c->host_out.data() + o0, (uint8_t *)c->out.p + o0, o1 - o0,
-			                                     hipMemcpyDeviceToHost, c->d2h_stream),
-			                      "D2H"))
-				return r;
+			if (int r = collect(next + 1 - kOutRing)) return r;
+			if (int r = hip_check(hipEventRecord(c->out_ev[next % kOutRing], c->stream), "hipEventRecord")) return r;
 			++next;
 		}
 		return 0;
 	};
-	if (int r = upload_large(c, c->src.p, src, n * srccomps, c->copy_stream, on_chunk)) return r;
+	if (int r = upload_chunks(c, crew, c->src.p, c->copy_stream[0], c->copy_stream[1], on_chunk)) return r;
 	if (next != nbands) return set_error(S2TC_E_ARG, "banded encode: %d of %d bands launched", next, nbands);
-	return hip_check(hipStreamSynchronize(c->d2h_stream), "hipStreamSynchronize");
+	while (back < nbands)
+		if (int r = collect(back + 1)) return r;
+	while (rows_dest && !crew.rows_copied())
+		if (!crew.step()) std::this_thread::yield();
+	return 0;
 }
 
 static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, const uint8_t *src, int dxt, int cd,
-                                int nrandom, int refine, int dither, uint64_t seed);
+                                int nrandom, int refine, int dither, uint64_t seed, uint8_t *rows_dest,
+                                size_t row_pitch, bool &rows_written);
 
 // Whole-image encode of host data on the context's stream; writes the
-// blocks in raster order to c->host_out.  On an error every stream of the
+// blocks in raster order to c->host_out, and their rows to rows_dest (if given)
+// where it says so in rows_written.  On an error every stream of the
 // context is drained before the context goes back to the pool, so that no
 // launch of this call still uses its buffers when the next call resizes them.
 static int encode_host_image(Ctx *c, int srccomps, int width, int height, const uint8_t *src, int dxt, int cd,
-                             int nrandom, int refine, int dither, uint64_t seed)
+                             int nrandom, int refine, int dither, uint64_t seed, uint8_t *rows_dest, size_t row_pitch,
+                             bool &rows_written)
 {
-	const int rc = encode_host_image_on(c, srccomps, width, height, src, dxt, cd, nrandom, refine, dither, seed);
+	const int rc = encode_host_image_on(c, srccomps, width, height, src, dxt, cd, nrandom, refine, dither, seed,
+	                                    rows_dest, row_pitch, rows_written);
 	if (rc) {
-		for (hipStream_t st : {c->stream, c->copy_stream, c->dither_stream, c->d2h_stream})
+		for (hipStream_t st : {c->stream, c->copy_stream[0], c->copy_stream[1]})
 			if (st) (void)hipStreamSynchronize(st);
 	}
 	return rc;
 }
 
 static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, const uint8_t *src, int dxt, int cd,
-                                int nrandom, int refine, int dither, uint64_t seed)
+                                int nrandom, int refine, int dither, uint64_t seed, uint8_t *rows_dest,
+                                size_t row_pitch, bool &rows_written)
 {
+	rows_written = false;
 	if (srccomps != 3) srccomps = 4;
 	if (dither != DITHER_NONE && dither != DITHER_FLOYDSTEINBERG) dither = DITHER_SIMPLE;
 	const size_t n = (size_t)width * height;
 	const size_t nb = (size_t)((width + 3) / 4) * ((height + 3) / 4);
 	const size_t obytes = nb * block_bytes(dxt);
 	const int alphabits = dxt == DXT1 ? 1 : dxt == DXT3 ? 4 : 8;
-	if (int r = c->src.ensure(n * srccomps)) return r;
-	if (int r = c->out.ensure(obytes)) return r;
+	const bool bands = dither != DITHER_FLOYDSTEINBERG && height > 8 && n * srccomps > kBandMin;
+	const bool direct = n * srccomps <= kDirectMax, direct_out = bands || obytes <= kDirectMax;
+	if (int r = direct ? c->in_stage.ensure(n * srccomps) : c->src.ensure(n * srccomps)) return r;
+	const void *d_src = direct ? c->in_stage.dev : c->src.p;
+	if (int r = c->host_out.ensure(obytes)) return r;
+	if (int r = direct_out ? 0 : c->out.ensure(obytes)) return r;
 	EncodeArgs a{};
-	a.dst = c->out.p;
+	a.dst = direct_out ? c->host_out.dev : c->out.p;
 	a.width = width;
 	a.height = height;
 	a.dxt = dxt;
@@ -361,29 +411,31 @@ static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, con
 	a.nrandom = nrandom;
 	a.refine = refine;
 	a.seed = seed;
-	if (dither != DITHER_FLOYDSTEINBERG && height > band_rows(width) && n * srccomps > kStageMax) {
-		// the blocks are in c->host_out once the last band's download is done
-		return encode_host_bands(c, srccomps, width, height, src, dxt, a, dither, alphabits);
-	} else {
-		if (int r = upload(c, c->src.p, src, n * srccomps)) return r;
-		if (dither == DITHER_NONE && srccomps == 4) {
-			a.src = c->src.p;  // quantization fused into the encoder's loads
-			a.src_kind = S2TC_SRC_RGBA8;
-		} else {
-			if (int r = c->q.ensure(n * 4)) return r;
-			if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height, dither))) return r;
-			if (int r = launch_rgb565(c->src.p, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p,
-			                          c->stream))
-				return r;
-			a.src = c->q.p;
-			a.src_kind = S2TC_SRC_QUANTIZED;
-		}
-		if (int r = launch_encode(a, c->stream)) return r;
+	if (bands) {
+		// the blocks are in c->host_out once the last band is encoded
+		if (int r = encode_host_bands(c, srccomps, width, height, src, dxt, a, dither, alphabits, rows_dest, row_pitch))
+			return r;
+		rows_written = rows_dest != nullptr;
+		return 0;
 	}
-	if (int r = c->host_out.ensure(obytes)) return r;
-	if (int r = hip_check(hipMemcpyAsync(c->host_out.data(), c->out.p, obytes, hipMemcpyDeviceToHost, c->stream),
-	                      "D2H"))
-		return r;
+	if (direct) memcpy(c->in_stage.p, src, n * srccomps);
+	else if (int r = upload(c, c->src.p, src, n * srccomps)) return r;
+	if (dither == DITHER_NONE && srccomps == 4) {
+		a.src = d_src;  // quantization fused into the encoder's loads
+		a.src_kind = S2TC_SRC_RGBA8;
+	} else {
+		if (int r = c->q.ensure(n * 4)) return r;
+		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height, dither))) return r;
+		if (int r = launch_rgb565(d_src, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p, c->stream))
+			return r;
+		a.src = c->q.p;
+		a.src_kind = S2TC_SRC_QUANTIZED;
+	}
+	if (int r = launch_encode(a, c->stream)) return r;
+	if (!direct_out)
+		if (int r = hip_check(hipMemcpyAsync(c->host_out.data(), c->out.p, obytes, hipMemcpyDeviceToHost, c->stream),
+		                      "D2H"))
+			return r;
 	return hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 }
 
@@ -496,37 +548,36 @@ void tx_compress_dxtn(GLint srccomps, GLint width, GLint height, const GLubyte *
 		fprintf(stderr, "s2tc: cannot create a HIP stream\n");
 		return;
 	}
-	if (int r = encode_host_image(g.c, srccomps, width, height, srcPixData, dxt, e.cd, e.nrandom, e.refine, e.dither,
-	                              e.seed)) {
-		fprintf(stderr, "s2tc: tx_compress_dxtn failed (%d): %s\n", r, s2tc_amd_last_error());
-		return;
-	}
 	// destination layout with dstRowDiff (s2tc_libtxc_dxtn.cpp:243, :261, :279)
 	const int bs = block_bytes(dxt);
 	const int bw = (width + 3) / 4, bh = (height + 3) / 4;
 	const long rowdiff = dstRowStride >= width * k ? (long)dstRowStride - (long)((width + 3) & ~3) * k : 0;
 	const size_t rowbytes = (size_t)bw * bs;
-	const uint8_t *hout = g.c->host_out.data();
-	auto copy_rows = [&](int lo, int hi) {
-		for (int by = lo; by < hi; ++by)
-			memcpy(dest + ((long)rowbytes + rowdiff) * by, hout + (size_t)by * rowbytes, rowbytes);
-	};
-	const unsigned hw = std::thread::hardware_concurrency();
-	const unsigned nt = std::max(1u, std::min(kUploadThreads, hw ? hw : 1u));
-	if (rowdiff < 0 || nt == 1 || rowbytes * (size_t)bh < (2u << 20)) {
-		// overlapping rows (a negative row gap) must be written in order
-		copy_rows(0, bh);
+	// rows that overlap each other (a negative row gap) are written in order, and
+	// rows over the source after the whole source is read
+	const uintptr_t s0 = (uintptr_t)srcPixData, s1 = s0 + (size_t)width * height * (srccomps == 3 ? 3 : 4);
+	const uintptr_t d0 = (uintptr_t)dest, d1 = d0 + (rowbytes + (size_t)std::max(rowdiff, 0L)) * (size_t)bh;
+	const bool early = rowdiff >= 0 && (d1 <= s0 || s1 <= d0);
+	bool written = false;
+	if (int r = encode_host_image(g.c, srccomps, width, height, srcPixData, dxt, e.cd, e.nrandom, e.refine, e.dither,
+	                              e.seed, early ? dest : nullptr, rowbytes + (size_t)rowdiff, written)) {
+		fprintf(stderr, "s2tc: tx_compress_dxtn failed (%d): %s\n", r, s2tc_amd_last_error());
 		return;
 	}
-	// disjoint rows: several host threads, contiguous row ranges each
-	std::vector<std::thread> workers;
-	const int per = (bh + (int)nt - 1) / (int)nt;
-	for (unsigned t = 1; t < nt; ++t) {
-		const int lo = std::min(bh, per * (int)t), hi = std::min(bh, lo + per);
-		if (hi > lo) workers.emplace_back(copy_rows, lo, hi);
+	if (written) return;
+	const uint8_t *hout = g.c->host_out.data();
+	if (rowdiff < 0 || rowbytes * (size_t)bh < (2u << 20)) {
+		for (int by = 0; by < bh; ++by)
+			memcpy(dest + ((long)rowbytes + rowdiff) * by, hout + (size_t)by * rowbytes, rowbytes);
+		return;
 	}
-	copy_rows(0, std::min(bh, per));
-	for (auto &w : workers) w.join();
+	// disjoint rows: several host threads
+	CopyCrew crew(nullptr, 0, nullptr, 1, 1);
+	crew.set_rows(dest, hout, rowbytes, rowbytes + (size_t)rowdiff, bh);
+	crew.open_rows(bh);
+	crew.start(copy_helpers());
+	while (!crew.rows_copied())
+		if (!crew.step()) std::this_thread::yield();
 }
 
 void rgb565_image(unsigned char *out, const unsigned char *rgba, int w, int h, int srccomps, int alphabits,
@@ -548,6 +599,7 @@ void rgb565_image(unsigned char *out, const unsigned char *rgba, int w, int h, i
 	if (!r) r = launch_rgb565(c->src.p, sc, w, h, alphabits, (int)dither, c->q.p, c->scratch.p, c->stream);
 	if (!r) r = hip_check(hipMemcpyAsync(out, c->q.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
 	if (!r) r = hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+	if (r) (void)hipStreamSynchronize(c->stream);
 	if (r) fprintf(stderr, "s2tc: rgb565_image failed (%d): %s\n", r, s2tc_amd_last_error());
 }
 
