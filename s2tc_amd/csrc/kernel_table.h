@@ -29,8 +29,7 @@ struct TileJobs {
 };
 
 struct KernelTable {
-	const void *fast[3][2];       // [dxt][raw]: k_fast_edge (partial blocks), null for NORMALMAP
-	const void *fast_int[3][2][3];  // [dxt][raw][refine]: k_fast_interior (full blocks), null for NORMALMAP
+	const void *fast[3][2][3][2];  // [dxt][raw][refine][edge]: k_fast_interior (full blocks; edge: and partial ones), null for NORMALMAP
 	const void *normal[2][2];     // [many][raw]: k_normal<CD, raw, RB> (many: normal_many)
 	const void *normal_wide[2];   // [raw]: k_normal_wide<CD, raw> (group memory in global scratch)
 	int normal_smem_cand;         // LDS bytes per candidate slot of a 4-block workgroup (candidate words)

@@ -97,54 +97,61 @@ template <int DXT> S2TC_D void store_block(uint8_t *dst, size_t b, const BlockOu
 	const size_t b = (size_t)by * (size_t)bw + (size_t)bx;                          \
 	const int w = min(4, width - 4 * bx), h = min(4, height - 4 * by);
 
-// Quick mode over the partial blocks of one image, one lane per block: the
-// bottom block row if height % 4 (ceil(width / 4) blocks), then the right
-// block column above it if width % 4.
-template <int CD, int DXT, bool RAW>
-__global__ __launch_bounds__(256, 4) void k_fast_edge(const uint32_t *__restrict__ src, int width, int height,
-                                                      uint8_t *__restrict__ dst, int refine)
+// Quick mode on a partial block of an image: block e of the bottom block row if
+// height % 4 (ceil(width / 4) blocks), then of the right block column above it
+// if width % 4.
+template <int CD, int DXT, bool RAW, int REFINE>
+S2TC_D void fast_edge_block(const uint32_t *__restrict__ src, int width, int height, uint8_t *__restrict__ dst, int e)
 {
+	const int refine = REFINE;
 	const int bw = (width + 3) >> 2, rows = height >> 2;
-	const int e = (int)(blockIdx.x * 256 + threadIdx.x), bottom = (height & 3) ? bw : 0;
+	const int bottom = (height & 3) ? bw : 0;
 	if (e >= bottom + ((width & 3) ? rows : 0)) return;
 	const int bx = e < bottom ? e : bw - 1, by = e < bottom ? rows : e - bottom;
 	const size_t b = (size_t)by * (size_t)bw + (size_t)bx;
 	const int w = min(4, width - 4 * bx), h = min(4, height - 4 * by);
 	uint32_t tx[16];
 	BlockOut o;
+	const uint32_t *blk = src + (size_t)(4 * by) * (size_t)width + 4 * bx;
 	if constexpr (QuadW<CD>::value) {
 		load_block<DXT, false>(src, width, bx, by, w, h, tx);
-		const uint32_t *blk = src + (size_t)(4 * by) * (size_t)width + 4 * bx;
 		o = encode_block_quad_any<CD, DXT, RAW>(tx, blk, width, w, h, refine);
+	} else if constexpr (LinW<CD>::value && REFINE != REFINE_LOOP) {
+		load_block<DXT, false>(src, width, bx, by, w, h, tx);
+		o = encode_block_lin_any<CD, DXT, RAW>(tx, blk, width, w, h, refine);
 	} else {
-		bool lin = false;
-		if constexpr (LinW<CD>::value) lin = refine != REFINE_LOOP;
-		if (lin) {
-			load_block<DXT, false>(src, width, bx, by, w, h, tx);
-			const uint32_t *blk = src + (size_t)(4 * by) * (size_t)width + 4 * bx;
-			if constexpr (LinW<CD>::value) o = encode_block_lin_any<CD, DXT, RAW>(tx, blk, width, w, h, refine);
-		} else {
-			load_block<DXT, RAW>(src, width, bx, by, w, h, tx);
-			o = encode_block_fast<CD, DXT>(tx, w, h, refine);
-		}
+		load_block<DXT, RAW>(src, width, bx, by, w, h, tx);
+		o = encode_block_fast<CD, DXT>(tx, w, h, refine);
 	}
 	store_block<DXT>(dst, b, o);
 }
 
-// Quick mode over the full 4x4 blocks of an image: blocks (bx, by) with
-// bx < nbx, by0 <= by < nby.  Without partial-block code the kernel needs far
-// fewer registers, so more waves hide the loads; the partial blocks go to
-// k_fast_edge.  Row loads are 16 bytes at any texel alignment, so that odd
-// widths run here too.  Measured (MI355X, 4093 x 2047 SRGB DXT5 LOOP): 75 us, and 15 us for the edge;
-// 108 us in a kernel for any block with a load per texel.
-template <int CD, int DXT, bool RAW, int REFINE>
-__global__ __launch_bounds__(256) void k_fast_interior(const uint32_t *__restrict__ src, int width, int nbx, int nby,
-                                                       uint8_t *__restrict__ dst, int by0)
+// Quick mode over the blocks of one image, one lane per block: the full 4x4
+// blocks (bx, by) with by0 <= by, and with EDGE, for sizes that 4 does not
+// divide, the partial ones in the first `erows` rows of the grid.  Without
+// partial-block code the kernel needs far fewer registers, so more waves hide
+// the loads; with it, the few long waves of the partial blocks run beside the
+// others instead of after them.  Row loads are 16 bytes at any texel alignment,
+// so that odd widths run here too.  At least three waves per SIMD: SRGB DXT5
+// LOOP took 175 registers.  Measured (MI355X, 4093 x 2047 SRGB DXT5 LOOP): 75
+// us; 89 us with the partial blocks in a launch of their own, 118 us in a kernel
+// for any block with a load per texel; 255 x 255 WAVG DXT1 ALWAYS: 3.4, 6.1 and
+// 7.6 us.
+template <int CD, int DXT, bool RAW, int REFINE, bool EDGE>
+__global__ __launch_bounds__(256, 3) void k_fast_interior(const uint32_t *__restrict__ src, int width, int height,
+                                                          uint8_t *__restrict__ dst, int by0, int erows)
 {
 	const int refine = REFINE;
+	const int row = (int)blockIdx.y - (EDGE ? erows : 0);
+	if (EDGE && row < 0) {
+		fast_edge_block<CD, DXT, RAW, REFINE>(src, width, height, dst,
+		                                      (int)((blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.y * 64 +
+		                                            threadIdx.x));
+		return;
+	}
 	const int bx = (int)(blockIdx.x * 64 + threadIdx.x);
-	const int by = by0 + (int)(blockIdx.y * 4 + threadIdx.y);
-	if (bx >= nbx || by >= nby) return;
+	const int by = by0 + row * 4 + (int)threadIdx.y;
+	if (bx >= width >> 2 || by >= height >> 2) return;
 	const size_t b = (size_t)by * (size_t)((width + 3) >> 2) + (size_t)bx;
 	const uint32_t *blk = src + (size_t)(4 * by) * (size_t)width + 4 * bx;
 	uint32_t tx[16];
@@ -611,23 +618,20 @@ using namespace s2tc;
 extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 {
 #if S2TC_CD != 7  /* NORMALMAP never runs in quick mode (s2tc_algorithm.cpp:1131-1134) */
-	kt->fast[DXT1][0] = (const void *)k_fast_edge<S2TC_CD, DXT1, false>;
-	kt->fast[DXT3][0] = (const void *)k_fast_edge<S2TC_CD, DXT3, false>;
-	kt->fast[DXT5][0] = (const void *)k_fast_edge<S2TC_CD, DXT5, false>;
-	kt->fast[DXT1][1] = (const void *)k_fast_edge<S2TC_CD, DXT1, true>;
-	kt->fast[DXT3][1] = (const void *)k_fast_edge<S2TC_CD, DXT3, true>;
-	kt->fast[DXT5][1] = (const void *)k_fast_edge<S2TC_CD, DXT5, true>;
-#define S2TC_INT3(D, R)                                                                      \
-	kt->fast_int[D][R][0] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_NEVER>;  \
-	kt->fast_int[D][R][1] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_ALWAYS>; \
-	kt->fast_int[D][R][2] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_LOOP>;
+#define S2TC_INT3(D, R)                                                                    \
+	kt->fast[D][R][0][0] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_NEVER, false>;  \
+	kt->fast[D][R][1][0] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_ALWAYS, false>; \
+	kt->fast[D][R][2][0] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_LOOP, false>;   \
+	kt->fast[D][R][0][1] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_NEVER, true>;   \
+	kt->fast[D][R][1][1] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_ALWAYS, true>;  \
+	kt->fast[D][R][2][1] = (const void *)k_fast_interior<S2TC_CD, D, R, REFINE_LOOP, true>;
 	S2TC_INT3(DXT1, false) S2TC_INT3(DXT3, false) S2TC_INT3(DXT5, false)
 	S2TC_INT3(DXT1, true) S2TC_INT3(DXT3, true) S2TC_INT3(DXT5, true)
 #undef S2TC_INT3
 #else
 	for (int d = 0; d < 3; ++d) {
-		kt->fast[d][0] = kt->fast[d][1] = nullptr;
-		for (int r = 0; r < 3; ++r) kt->fast_int[d][0][r] = kt->fast_int[d][1][r] = nullptr;
+		for (int r = 0; r < 3; ++r)
+			kt->fast[d][0][r][0] = kt->fast[d][0][r][1] = kt->fast[d][1][r][0] = kt->fast[d][1][r][1] = nullptr;
 	}
 #endif
 #if S2TC_CD != 7

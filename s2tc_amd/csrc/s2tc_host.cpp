@@ -124,29 +124,35 @@ int launch_encode(const EncodeArgs &a, hipStream_t stream, void *ext_scratch, si
 	const void *src = a.src;
 	void *dst = a.dst;
 	int width = a.width, height = a.height;
-	if (is_fast(cd, a.nrandom) || a.nrandom <= 0) {
-		// one lane per block: quick mode, or only the block's colours
-		const bool fast = is_fast(cd, a.nrandom);
-		const void *k = fast ? kt.fast_int[dxt][raw][refine] : kt.all16[dxt][raw];
+	// one lane per block: quick mode, or only the block's colours
+	const dim3 block(64, 4);
+	const int rows_per_launch = 4 * 65000;  // grid.y limit of 65535 workgroups of 4 block rows
+	if (is_fast(cd, a.nrandom)) {
+		const void *const *k = kt.fast[dxt][raw][refine];
+		if (!k[0]) return set_error(S2TC_E_ARG, "no one-lane kernel for distance %d", cd);
+		const int nbx = width / 4, nby = height / 4, gx = (nbx + 63) / 64;
+		const int edge = ((height & 3) ? (width + 3) / 4 : 0) + ((width & 3) ? nby : 0);
+		const auto launch = [&](int grid_x, int by0, int erows, int brows) {
+			void *args[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&by0, (void *)&erows};
+			const dim3 grid((unsigned)grid_x, (unsigned)(erows + (brows + 3) / 4));
+			return hip_check(hipLaunchKernel(k[erows > 0], grid, block, args, 0, stream), "launch k_fast_interior");
+		};
+		// the partial blocks run with the full ones, unless there are none, or so
+		// many (tall and narrow) that grid.y would not hold their rows
+		int erows = nbx > 0 && nby > 0 ? (int)((edge + 256LL * gx - 1) / (256LL * gx)) : 0;
+		if (erows > 500) erows = 0;
+		for (int by0 = 0; nbx > 0 && by0 < nby; by0 += rows_per_launch)
+			if (int r = launch(gx, by0, by0 ? 0 : erows, std::min(nby - by0, rows_per_launch))) return r;
+		return edge && !erows ? launch((edge + 255) / 256, 0, 1, 0) : 0;
+	}
+	if (a.nrandom <= 0) {
+		const void *k = kt.all16[dxt][raw];
 		if (!k) return set_error(S2TC_E_ARG, "no one-lane kernel for distance %d", cd);
-		// quick mode: the full blocks, then the partial ones in a launch of their own
-		int nbx = fast ? width / 4 : (width + 3) / 4, nby = fast ? height / 4 : (height + 3) / 4;
-		const int rows_per_launch = 4 * 65535;  // grid.y limit of 65535 workgroups of 4 block rows
-		for (int by0 = 0; nbx > 0 && by0 < nby; by0 += rows_per_launch) {
-			const int rows = nby - by0 < rows_per_launch ? nby - by0 : rows_per_launch;
-			void *fargs[] = {(void *)&src, (void *)&width, (void *)&nbx, (void *)&nby, (void *)&dst, (void *)&by0};
-			void *nargs[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&refine, (void *)&by0};
-			dim3 grid((unsigned)((nbx + 63) / 64), (unsigned)((rows + 3) / 4)), block(64, 4);
-			if (int r = hip_check(hipLaunchKernel(k, grid, block, fast ? fargs : nargs, 0, stream),
-			                      "launch one-lane encoder"))
-				return r;
-		}
-		const int edge = fast ? ((height & 3) ? (width + 3) / 4 : 0) + ((width & 3) ? height / 4 : 0) : 0;
-		if (edge) {
-			void *args[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&refine};
-			return hip_check(hipLaunchKernel(kt.fast[dxt][raw], dim3((unsigned)((edge + 255) / 256)), dim3(256), args, 0,
-			                                 stream),
-			                 "launch k_fast_edge");
+		const int nbx = (width + 3) / 4, nby = (height + 3) / 4;
+		for (int by0 = 0; by0 < nby; by0 += rows_per_launch) {
+			void *args[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&refine, (void *)&by0};
+			const dim3 grid((unsigned)((nbx + 63) / 64), (unsigned)((std::min(nby - by0, rows_per_launch) + 3) / 4));
+			if (int r = hip_check(hipLaunchKernel(k, grid, block, args, 0, stream), "launch k_all16")) return r;
 		}
 		return 0;
 	}
@@ -155,12 +161,12 @@ int launch_encode(const EncodeArgs &a, hipStream_t stream, void *ext_scratch, si
 	unsigned long long seed = a.seed;
 	unsigned block_base = a.block_index_base;
 	if (nrandom <= S2TC_LDS_NRANDOM) {
-		dim3 grid((unsigned)((nb + 3) / 4)), block(64);
+		dim3 grid((unsigned)((nb + 3) / 4));
 		const bool many = normal_many(pbw, grid.x);
 		size_t smem = normal_group_smem(kt, pbw, many);
 		void *args[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&dxt,
 		                (void *)&nrandom, (void *)&refine, (void *)&seed, (void *)&pbw, (void *)&block_base};
-		return hip_check(hipLaunchKernel(kt.normal[many][raw], grid, block, args, smem, stream), "launch k_normal");
+		return hip_check(hipLaunchKernel(kt.normal[many][raw], grid, dim3(64), args, smem, stream), "launch k_normal");
 	}
 	// more candidates than LDS holds: group memory in the caller's scratch, or
 	// in stream-ordered scratch that lives exactly as long as this launch
