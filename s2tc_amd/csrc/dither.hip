@@ -232,7 +232,7 @@ template <int ALPHA> constexpr int table_words() { return ALPHA == ALPHA_4 ? 768
 // The workgroup's cnt texels from src as words {r, g, b, a} (a = 0 for three
 // components); the words past them, up to `room`, are 0.
 template <int COMPS>
-__device__ __forceinline__ void load_texels(const uint8_t *__restrict__ src, int cnt, int room, int lsh, uint32_t *tex)
+__device__ __forceinline__ void load_texels(const uint8_t *src, int cnt, int room, int lsh, uint32_t *tex)
 {
 	const uint32_t *g = (const uint32_t *)src;
 	for (int q = (int)threadIdx.x; 4 * q < room; q += (int)blockDim.x) {
@@ -336,15 +336,16 @@ __device__ __forceinline__ void emit_chunk(uint32_t *tex, int len, uint32_t stat
 }
 
 // The workgroup's first cnt words to out.
-__device__ __forceinline__ void store_texels(const uint32_t *tex, int cnt, int lsh, uint32_t *__restrict__ out)
+__device__ __forceinline__ void store_texels(const uint32_t *tex, int cnt, int lsh, uint32_t *out)
 {
 	for (int i = (int)threadIdx.x; i < cnt; i += (int)blockDim.x) out[i] = tex[i + (i >> lsh)];
 }
 
-// Maps of the workgroup's chunks and waves.
+// Maps of the workgroup's chunks and waves.  raw (may be null): takes the
+// texels as words.
 template <int COMPS, int ALPHA>
 __global__ __launch_bounds__(SIMPLE_WG) void k_simple_maps(const uint8_t *__restrict__ src, long long n, int lsh,
-                                                           SimpleScratch s)
+                                                           SimpleScratch s, uint32_t *__restrict__ raw)
 {
 	uint32_t *tab = simple_lds, *tex = simple_lds + table_words<ALPHA>();
 	const int L = 1 << lsh;
@@ -353,6 +354,7 @@ __global__ __launch_bounds__(SIMPLE_WG) void k_simple_maps(const uint8_t *__rest
 	for (int i = (int)threadIdx.x; i < table_words<ALPHA>(); i += SIMPLE_WG) tab[i] = c_entries.t[i];
 	load_texels<COMPS>(src + p0 * COMPS, cnt, SIMPLE_WG << lsh, lsh, tex);
 	__syncthreads();
+	if (raw) store_texels(tex, cnt, lsh, raw + p0);
 	Maps<ALPHA> m;
 	chunk_maps<ALPHA>(tex + (int)threadIdx.x * (L + 1), min(L, max(0, cnt - ((int)threadIdx.x << lsh))), tab, m);
 	wave_scan(m.r);
@@ -448,11 +450,12 @@ __device__ __forceinline__ uint32_t scan_here(const uint32_t *maps, int nw, int 
 	}
 }
 
+// src may be out: a workgroup has read its texels before it writes them.
 template <int COMPS, int ALPHA>
-__global__ __launch_bounds__(SIMPLE_WG) void k_simple_emit(const uint8_t *__restrict__ src, long long n, int lsh,
-                                                           int plain, SimpleScratch s, int scan,
+__global__ __launch_bounds__(SIMPLE_WG) void k_simple_emit(const uint8_t *src, long long n, int lsh, int plain,
+                                                           SimpleScratch s, int scan,
                                                            const uint8_t *__restrict__ carry_in,
-                                                           uint8_t *__restrict__ carry_out, uint32_t *__restrict__ out)
+                                                           uint8_t *__restrict__ carry_out, uint32_t *out)
 {
 	uint32_t *tex = simple_lds;
 	const int lane = (int)(threadIdx.x & 63), L = 1 << lsh;
@@ -584,7 +587,7 @@ size_t rgb565_scratch_bytes(int w, int h, int dither)
 
 template <int COMPS, int ALPHA>
 static int run_simple(const uint8_t *src, long long n, int plain, void *scr, const uint8_t *carry_in,
-                      uint8_t *carry_out, uint32_t *out, hipStream_t st)
+                      uint8_t *carry_out, uint32_t *out, hipStream_t st, bool host_src)
 {
 	const size_t tab = (size_t)table_words<ALPHA>() * 4;
 	if (n <= SIMPLE_ONE) {
@@ -614,10 +617,17 @@ static int run_simple(const uint8_t *src, long long n, int plain, void *scr, con
 	const int lsh = simple_lsh(n), scan = s.nw <= 64;
 	const unsigned grid = (unsigned)((s.nw + SIMPLE_WG / 64 - 1) / (SIMPLE_WG / 64));
 	const size_t lds = (size_t)SIMPLE_WG * ((1 << lsh) + 1) * 4;
-	k_simple_maps<COMPS, ALPHA><<<grid, SIMPLE_WG, tab + lds, st>>>(src, n, lsh, s);
+	// a source in host memory crosses the bus once: the first kernel leaves its
+	// texels where the last one writes the quantized ones (256 x 256 calls 41 ->
+	// 36 us; in device memory reading them twice costs less than the writes)
+	k_simple_maps<COMPS, ALPHA><<<grid, SIMPLE_WG, tab + lds, st>>>(src, n, lsh, s, host_src ? out : nullptr);
 	if (!scan)
 		k_simple_states<ALPHA><<<ALPHA == ALPHA_PLAIN ? 3 : 4, 1024, 0, st>>>(s, carry_in, carry_out);
-	k_simple_emit<COMPS, ALPHA><<<grid, SIMPLE_WG, lds, st>>>(src, n, lsh, plain, s, scan, carry_in, carry_out, out);
+	if (host_src)
+		k_simple_emit<4, ALPHA><<<grid, SIMPLE_WG, lds, st>>>((const uint8_t *)out, n, lsh, plain, s, scan, carry_in,
+		                                                      carry_out, out);
+	else
+		k_simple_emit<COMPS, ALPHA><<<grid, SIMPLE_WG, lds, st>>>(src, n, lsh, plain, s, scan, carry_in, carry_out, out);
 	return hip_check(hipGetLastError(), "dither SIMPLE kernels");
 }
 
@@ -626,7 +636,7 @@ static int run_simple(const uint8_t *src, long long n, int plain, void *scr, con
 // (:1437-1449), dither other than NONE and FLOYDSTEINBERG means SIMPLE
 // (:1419-1431).
 int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, int dither, void *d_out,
-                  void *d_scratch, hipStream_t st, const void *d_carry_in, void *d_carry_out)
+                  void *d_scratch, hipStream_t st, const void *d_carry_in, void *d_carry_out, bool host_src)
 {
 	if (srccomps != 3) srccomps = 4;
 	if (alphabits != 1 && alphabits != 4) alphabits = 8;
@@ -646,10 +656,10 @@ int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, 
 	}
 	const uint8_t *ci = (const uint8_t *)d_carry_in;
 	uint8_t *co = (uint8_t *)d_carry_out;
-	if (srccomps == 3) return run_simple<3, ALPHA_PLAIN>(src, n, (1 << alphabits) - 1, d_scratch, ci, co, out, st);
-	if (alphabits == 1) return run_simple<4, ALPHA_MOD>(src, n, 0, d_scratch, ci, co, out, st);
-	if (alphabits == 4) return run_simple<4, ALPHA_4>(src, n, 0, d_scratch, ci, co, out, st);
-	return run_simple<4, ALPHA_PLAIN>(src, n, -1, d_scratch, ci, co, out, st);
+	if (srccomps == 3) return run_simple<3, ALPHA_PLAIN>(src, n, (1 << alphabits) - 1, d_scratch, ci, co, out, st, host_src);
+	if (alphabits == 1) return run_simple<4, ALPHA_MOD>(src, n, 0, d_scratch, ci, co, out, st, host_src);
+	if (alphabits == 4) return run_simple<4, ALPHA_4>(src, n, 0, d_scratch, ci, co, out, st, host_src);
+	return run_simple<4, ALPHA_PLAIN>(src, n, -1, d_scratch, ci, co, out, st, host_src);
 }
 
 }  // namespace s2tc

@@ -53,9 +53,12 @@ int launch_pull(void *dst, const void *src, size_t n, hipStream_t st);
 // band of rows of a larger one, which starts from the error states in
 // d_carry_in (null: from the reference's initial ones) and leaves its end
 // states in d_carry_out for the next band.
+// host_src: d_src is pinned host memory, worth reading once only; d_out is then
+// 16-byte aligned.
 size_t rgb565_scratch_bytes(int w, int h, int dither);
 int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, int dither, void *d_out,
-                  void *d_scratch, hipStream_t st, const void *d_carry_in = nullptr, void *d_carry_out = nullptr);
+                  void *d_scratch, hipStream_t st, const void *d_carry_in = nullptr, void *d_carry_out = nullptr,
+                  bool host_src = false);
 
 // The Floyd-Steinberg dither (dither_fs.hip), arguments normalised.
 size_t rgb565_fs_scratch_bytes(int w, int h);

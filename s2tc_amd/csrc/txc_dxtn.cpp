@@ -73,8 +73,8 @@ struct HostBuf {
 // back and the rows laid out, one after the other):
 //   up to kDirectMax, the kernels read the pinned copy of the source, and write
 //   blocks of up to kDirectMax to pinned memory: 256 x 256 RGBA quick 36 -> 21
-//   us, with the SIMPLE dither 50 -> 41 us (two passes over the bus still beat
-//   a DMA at 512 KiB, and lose at 1 MiB);
+//   us, with the SIMPLE dither 50 -> 36 us (at 1 MiB the Floyd-Steinberg dither
+//   loses: 189 -> 266 us for its short reads, the others change little);
 //   up to kBandMin, the upload kernel runs over each half while the other is
 //   copied: 1024 x 1024 SIMPLE 216 -> 175 us (four pieces: the same);
 //   above, in bands (encode_host_bands) with uploads of kChunk through a ring of
@@ -426,7 +426,8 @@ static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, con
 	} else {
 		if (int r = c->q.ensure(n * 4)) return r;
 		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height, dither))) return r;
-		if (int r = launch_rgb565(d_src, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p, c->stream))
+		if (int r = launch_rgb565(d_src, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p, c->stream,
+		                          nullptr, nullptr, direct))
 			return r;
 		a.src = c->q.p;
 		a.src_kind = S2TC_SRC_QUANTIZED;

@@ -49,6 +49,12 @@ def test_sizes(call, sc, w, h, dither):
     call(sc, w, h, 0x83F1 if w & 1 else 0x83F3, dither, gap=0 if h & 2 else 48)
 
 
+@pytest.mark.parametrize("fmt", [0x83F0, 0x83F2, 0x83F3])
+@pytest.mark.parametrize("sc,w,h", [(4, 129, 65), (3, 129, 65), (3, 400, 437), (4, 361, 363)])
+def test_simple_from_pinned_memory(call, sc, w, h, fmt):
+    call(sc, w, h, fmt, 1)
+
+
 @pytest.mark.parametrize("sc,w,h,dither", [(4, 300001, 7, 1), (4, 240001, 9, 1), (3, 300000, 10, 0), (4, 120001, 19, 0),
                                            (4, 5, 500001, 1)])
 def test_bands_of_extreme_shapes(call, sc, w, h, dither):
