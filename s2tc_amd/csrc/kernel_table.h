@@ -35,7 +35,7 @@ struct KernelTable {
 	int normal_smem_cand;         // LDS bytes per candidate slot of a 4-block workgroup (candidate words)
 	int normal_smem_fixed;        // plus these bytes (features of the 16 texel candidates of 4 blocks)
 	const void *fast_batch[3][3]; // [dxt][refine]: persistent quick-mode kernel over a job list
-	const void *normal_batch[2];  // [many]: persistent MODE_NORMAL kernel over a job list
+	const void *normal_batch;     // persistent MODE_NORMAL kernel over a job list
 	const void *normal_batch_wide;  // the same with group memory in global scratch
 	const void *all16[3][2];      // [dxt][raw]: MODE_NORMAL without random colours, one lane per block
 	const void *all16_batch[3][3];  // [dxt][refine]: its persistent batch form
@@ -55,6 +55,10 @@ struct KernelTable {
 // 278 us and 1075 -> 975 us.  Outside that range, and where a launch has no
 // more workgroups than eight to a CU, the third row block only costs moves:
 // 48 random colours up to 8% slower, 128 SRGB 2%, 256 x 256 SRGB 8%.
+// The batch kernel always has two: its class takes textures of all counts, and
+// 40 textures of 256 x 256 with 8 random colours beside one with 64 took 401 us
+// with two and 456 us with three (SRGB), 40 with 64 1314 and 1350 us; RGB, YUV
+// and SRGB_MIXED alike, and the other distances gain nothing.
 #define S2TC_RB_FEW 2
 #define S2TC_RB_MANY 3
 inline bool normal_many(int pbw, long long workgroups)

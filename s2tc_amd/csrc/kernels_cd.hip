@@ -462,14 +462,14 @@ S2TC_D BlockIn fetch_block(const JobDesc *__restrict__ jobs, TileJobs tj, int ti
 	return in;
 }
 
-template <int CD, int RB> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<CD> &sm, int t)
+template <int CD> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<CD> &sm, int t)
 {
 	const int x = t >> 2, y = t & 3;
 	uint32_t tex = 0;
 	if (x < in.w && y < in.h) tex = in.raw ? quant_none_rt(in.tex, in.dxt) : in.tex;
 	const int pbw = (16 + (in.nrandom > 0 ? in.nrandom : 0) + 15) / 16;
 	BlockOut o;
-	encode_block_normal<CD, RB, true>(tex, t, in.w, in.h, in.dxt, in.nrandom, in.refine, in.bkey, pbw, sm, o);
+	encode_block_normal<CD, S2TC_RB_FEW, true>(tex, t, in.w, in.h, in.dxt, in.nrandom, in.refine, in.bkey, pbw, sm, o);
 	if (in.have && t == 0) {
 		if (in.dxt == DXT1) store_block<DXT1>(in.dst, (size_t)in.b, o);
 		else store_block<DXT5>(in.dst, (size_t)in.b, o);
@@ -480,14 +480,14 @@ template <int CD, int RB> S2TC_D void encode_fetched(const BlockIn &in, const Gr
 // job and texels of tile T + G are in flight and the tile record of T + 2G
 // (G = grid size; indices past the end are clamped to the last tile, whose
 // inputs are then fetched and never used).
-template <int CD, int RB>
-__global__ __launch_bounds__(64) S2TC_RB_WAVES(RB) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
+template <int CD>
+__global__ __launch_bounds__(64) S2TC_RB_WAVES(S2TC_RB_FEW) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
                                                      long long nblocks, int ntiles, int pbw_max)
 {
 	extern __shared__ __align__(16) uint8_t smem[];
 	const int lane = (int)threadIdx.x;
 	const int g = lane >> 4, t = lane & 15;
-	const GroupSmem<CD> sm = group_smem<CD, RB>(smem, g, 16 * pbw_max);
+	const GroupSmem<CD> sm = group_smem<CD, S2TC_RB_FEW>(smem, g, 16 * pbw_max);
 	const int G = (int)gridDim.x;
 	int tile = xcd_local_id((int)blockIdx.x, G);
 	if (tile >= ntiles) return;
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(64) S2TC_RB_WAVES(RB) void k_normal_batch(const Job
 	for (; tile < ntiles; tile += G) {
 		const BlockIn nxt = fetch_block(jobs, tjn, min(tile + G, ntiles - 1), nblocks, g, t);
 		tjn = tile_at(tile + 2 * G);
-		encode_fetched<CD, RB>(cur, sm, t);
+		encode_fetched<CD>(cur, sm, t);
 		__syncthreads();
 		cur = nxt;
 	}
@@ -644,8 +644,7 @@ extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 #else
 	for (int d = 0; d < 3; ++d) kt->fast_batch[d][0] = kt->fast_batch[d][1] = kt->fast_batch[d][2] = nullptr;
 #endif
-	kt->normal_batch[0] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_FEW>;
-	kt->normal_batch[1] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_MANY>;
+	kt->normal_batch = (const void *)k_normal_batch<S2TC_CD>;
 	kt->normal_batch_wide = (const void *)k_normal_batch_wide<S2TC_CD>;
 	kt->error[DXT1][0] = (const void *)k_colordist_error<S2TC_CD, DXT1, false>;
 	kt->error[DXT3][0] = (const void *)k_colordist_error<S2TC_CD, DXT3, false>;

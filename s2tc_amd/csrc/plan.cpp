@@ -108,13 +108,12 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 	for (auto &c : classes) {
 		const KernelTable &kt = kernel_table(c.cd);
 		c.ntiles = (int)((c.nblocks + c.tile - 1) / c.tile);
-		const bool many = normal_many(c.pbw_max, c.ntiles);
 		c.kernel = c.wide     ? kt.normal_batch_wide
-		           : c.normal ? kt.normal_batch[many]
+		           : c.normal ? kt.normal_batch
 		           : c.all16  ? kt.all16_batch[c.dxt][c.refine]
 		                      : kt.fast_batch[c.dxt][c.refine];
 		if (!c.kernel) return set_error(S2TC_E_ARG, "no batch kernel for distance %d", c.cd);
-		c.smem = c.normal && !c.wide ? normal_group_smem(kt, c.pbw_max, many) : 0;
+		c.smem = c.normal && !c.wide ? normal_group_smem(kt, c.pbw_max, false) : 0;
 		if (c.wide) wide_launch_shape(kt, c.pbw_max, c.ntiles, device_cu_count(), c.wide_grid, c.scratch);
 		tile_ranges(c.jobs, c.nblocks, c.tile, c.ntiles, c.tiles);
 		if (c.all16) {
@@ -123,7 +122,7 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 			c.forms[FORM_LANE_2WAVES] = k2 != c.kernel ? k2 : nullptr;
 			if (with_forms) {
 				// the random-candidate kernel runs nrandom-0 jobs as they are
-				c.forms[FORM_ROW16] = kt.normal_batch[0];
+				c.forms[FORM_ROW16] = kt.normal_batch;
 				c.ntiles4 = (int)((c.nblocks + 3) / 4);
 				c.smem4 = normal_group_smem(kt, 1, false);
 				tile_ranges(c.jobs, c.nblocks, 4, c.ntiles4, c.tiles4);
