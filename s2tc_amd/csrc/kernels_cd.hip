@@ -241,6 +241,12 @@ S2TC_D void normal_image_tile(const uint32_t *__restrict__ src, int width, int h
 // three row blocks in registers (kernel_table.h says why), else four (left to
 // itself the compiler spares registers for a fifth: SRGB scans 4% slower).
 #define S2TC_RB_WAVES(RB) __attribute__((amdgpu_waves_per_eu(RB == S2TC_RB_MANY ? 3 : 4, RB == S2TC_RB_MANY ? 3 : 4)))
+// The batch kernel also holds the next tile's inputs, which four waves a SIMD
+// leave no registers for: it would keep 28 to 108 bytes a lane in scratch (40
+// textures of 256 x 256, 16 random colours: RGB 327 us, 277 us without).  Three
+// waves; RGB and YUV in the registers that they take by themselves (told of
+// three, they come out 4% slower, the other distances up to 2% faster).
+#define S2TC_BATCH_WAVES(CD) __attribute__((amdgpu_waves_per_eu(CD <= CD_YUV ? 1 : 3, CD <= CD_YUV ? 8 : 3)))
 
 // Candidates, rows and column features in LDS (nrandom <= S2TC_LDS_NRANDOM);
 // one workgroup per tile.
@@ -481,7 +487,7 @@ template <int CD> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<
 // (G = grid size; indices past the end are clamped to the last tile, whose
 // inputs are then fetched and never used).
 template <int CD>
-__global__ __launch_bounds__(64) S2TC_RB_WAVES(S2TC_RB_FEW) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
+__global__ __launch_bounds__(64) S2TC_BATCH_WAVES(CD) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
                                                      long long nblocks, int ntiles, int pbw_max)
 {
 	extern __shared__ __align__(16) uint8_t smem[];
