@@ -608,7 +608,7 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 	bool dd = false;         // repeated colours are dropped from the colour scan (DEDUP)
 	uint32_t *ul = nullptr;
 	int V = 1;
-	const int cap = sm.ints;
+	const int cap = normal_table_ints(pbw, sm.ints);
 	if (nrandom > 0) {  // (:962-993)
 		const int r = c_r(v), g = c_g(v), b = c_b(v);
 		int minr = row_min(use ? r : 255), ming = row_min(use ? g : 255), minb = row_min(use ? b : 255);

@@ -83,6 +83,19 @@ S2TC_HD inline int normal_row_ints(int pbw, int rb)
 	return rb == S2TC_RB_MANY && rows < 560 ? 560 : rows;
 }
 
+// Ints of a block's row memory (`ints` in all) that the tables of the scan over
+// distinct colours and its list may take: no more than the rows of the block's
+// own pbw row blocks with two in registers, also where the launch was sized for
+// larger blocks of its class.  Blocks with few candidates have little to gain:
+// 40 textures with 16 random colours and 10 with 64 (256 x 256, NORMALMAP, boxes
+// of 30 to 250 cells) took 651 us with tables in all that the class has, 576 us
+// so; RGB 654 and 592 us.
+S2TC_HD inline int normal_table_ints(int pbw, int ints)
+{
+	const int own = 256 * (pbw > S2TC_RB_FEW ? pbw - S2TC_RB_FEW : 0);
+	return own < ints ? own : ints;
+}
+
 // Group memory of a four-block workgroup of the random-candidate kernels
 // with pbw row blocks: 16 pbw candidate slots, the row memory and the texel
 // features.

@@ -1,0 +1,33 @@
+// Host checks of the sizes of the random-candidate kernels' group memory
+// (kernel_table.h), compiled with g++ by tests/test_table_sizes.py.
+#include <cstdio>
+#include <initializer_list>
+
+#include "kernel_table.h"
+
+int main()
+{
+	for (int rb : {S2TC_RB_FEW, S2TC_RB_MANY})
+		for (int pbw_max = 1; pbw_max <= 14; ++pbw_max) {
+			const int ints = normal_row_ints(pbw_max, rb);
+			for (int pbw = 1; pbw <= pbw_max; ++pbw) {
+				const int t = normal_table_ints(pbw, ints);
+				// within the memory that there is, and for a block of few candidates
+				// as if its class had no larger ones
+				if (t < 0 || t > ints || (rb == S2TC_RB_FEW && t != normal_row_ints(pbw, rb))) {
+					printf("tables: %d of %d row blocks, %d in registers: %d of %d ints\n", pbw, pbw_max, rb, t, ints);
+					return 1;
+				}
+				if (pbw <= 2 && t != 0) {
+					printf("tables for %d row blocks\n", pbw);
+					return 1;
+				}
+			}
+			if (rb == S2TC_RB_MANY && pbw_max >= 5 && normal_table_ints(pbw_max, ints) != ints) {
+				printf("one image, %d row blocks: %d of %d ints\n", pbw_max, normal_table_ints(pbw_max, ints), ints);
+				return 1;
+			}
+		}
+	printf("ok\n");
+	return 0;
+}
