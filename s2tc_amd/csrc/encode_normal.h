@@ -576,7 +576,7 @@ template <int CD> struct PlainScan {
 // is bound by vector instructions.  Measured (MI355X, 4096 x 4096 smooth normal
 // map, 64 random colours, LOOP): 501 us, 802 us with three passes over the
 // candidates for the list and two register row blocks.
-template <int CD, int RB, bool DEDUP>
+template <int CD, int RB, bool DEDUP, bool CLEAR = false>
 S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int nrandom, int refine, uint32_t bkey,
                                 int pbw, const GroupSmem<CD> &sm, BlockOut &o)
 {
@@ -764,10 +764,10 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 			dv[k] = d;
 		}
 		// columns that are no candidates count nothing; rows that are none are
-		// never asked for
-		if (!whole) {
+		// never asked for (CLEAR: they are cleared as well)
+		if (CLEAR || !whole) {
 #pragma unroll
-			for (int k = 0; k < 16; ++k) dv[k] = k < n ? dv[k] : 0;
+			for (int k = 0; k < 16; ++k) dv[k] = k < n && (!CLEAR || irow) ? dv[k] : 0;
 		}
 		put_rows(sm.rows, R, p, t, dv);
 		if (dd && irow) {
