@@ -3,10 +3,12 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -28,9 +30,13 @@ inline void stage_slice(size_t len, unsigned nt, unsigned t, size_t &lo, size_t 
 // helpers take one by one: first those of the source (chunks of `chunk` bytes
 // into a ring of `ring` pinned buffers), then those of the block rows that came
 // back.  A slice can only be taken once its chunk or its rows are opened by the
-// calling thread, which alone talks to the GPU.
+// calling thread, which alone talks to the GPU.  Helpers that find no open slice
+// for a while sleep until one is opened: a call may wait long for its encoder.
 struct CopyCrew {
 	static const unsigned kParts = 8;  // slices per chunk
+	// Unsuccessful looks (about 50 us of yields, two chunks' uploads) before a
+	// helper sleeps; waking one takes about as long.
+	static const unsigned kIdle = 128;
 
 	const uint8_t *src;
 	uint8_t *stage;
@@ -45,6 +51,9 @@ struct CopyCrew {
 	std::atomic<size_t> out_next{0}, out_open{0}, out_done{0};
 
 	std::atomic<bool> quit{false};
+	std::atomic<unsigned> asleep{0};
+	std::mutex mu;
+	std::condition_variable opened;
 	std::vector<std::thread> helpers;
 
 	CopyCrew(const uint8_t *src_, size_t n_, uint8_t *stage_, size_t chunk_, size_t ring_)
@@ -75,16 +84,14 @@ struct CopyCrew {
 		try {
 			helpers.reserve(count);
 			for (unsigned t = 0; t < count; ++t)
-				helpers.emplace_back([this] {
-					while (!quit.load(std::memory_order_acquire))
-						if (!step()) std::this_thread::yield();
-				});
+				helpers.emplace_back([this] { help(); });
 		} catch (const std::exception &) {
 		}
 	}
 	void finish()
 	{
-		quit.store(true, std::memory_order_release);
+		quit.store(true);
+		wake();
 		for (auto &h : helpers) h.join();
 		helpers.clear();
 	}
@@ -92,12 +99,17 @@ struct CopyCrew {
 	size_t ring_offset(size_t i) const { return i % ring * chunk; }
 	size_t chunk_len(size_t i) const { return std::min(chunk, n - i * chunk); }
 	// chunks before `i` may be copied (their buffers are free)
-	void open_chunks(size_t i) { up_open.store(i * kParts, std::memory_order_release); }
+	void open_chunks(size_t i)
+	{
+		up_open.store(i * kParts);
+		wake();
+	}
 	bool chunk_copied(size_t i) const { return done[i].load(std::memory_order_acquire) == kParts; }
 	// block rows before `rows` have come back
 	void open_rows(int rows)
 	{
-		out_open.store(rows >= nrows ? out_slices() : (size_t)(rows / rows_per_slice), std::memory_order_release);
+		out_open.store(rows >= nrows ? out_slices() : (size_t)(rows / rows_per_slice));
+		wake();
 	}
 	bool rows_copied() const { return out_done.load(std::memory_order_acquire) == out_slices(); }
 
@@ -124,6 +136,33 @@ struct CopyCrew {
 	}
 
 private:
+	bool has_work() const { return quit.load() || up_next.load() < up_open.load() || out_next.load() < out_open.load(); }
+	// A helper counts itself asleep before it looks for work the last time, and
+	// whoever opens slices looks for sleepers afterwards, both in the one order of
+	// the sequentially consistent operations: one of the two sees the other.
+	void wake()
+	{
+		if (!asleep.load()) return;
+		std::lock_guard<std::mutex> lk(mu);
+		opened.notify_all();
+	}
+	void help()
+	{
+		unsigned idle = 0;
+		while (!quit.load(std::memory_order_acquire)) {
+			if (step()) {
+				idle = 0;
+			} else if (++idle < kIdle) {
+				std::this_thread::yield();
+			} else {
+				std::unique_lock<std::mutex> lk(mu);
+				++asleep;
+				opened.wait(lk, [this] { return has_work(); });
+				--asleep;
+				idle = 0;
+			}
+		}
+	}
 	static bool take(std::atomic<size_t> &next, const std::atomic<size_t> &open, size_t &i)
 	{
 		i = next.load(std::memory_order_relaxed);
