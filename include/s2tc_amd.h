@@ -250,7 +250,7 @@ typedef struct {
 S2TC_API int s2tc_amd_serve(const s2tc_amd_job *jobs, int njobs, const s2tc_amd_request *reqs, int nreq,
                             const s2tc_amd_serve_opts *opts, double *latency_ms, s2tc_amd_serve_stats *stats);
 
-/* ---- test hook ---- */
+/* ---- test hooks ---- */
 
 /* No counterpart in the reference; for tests only.  The pair scan of the
  * random-candidate encoder under RGB, YUV and SRGB_MIXED keys its pair sums
@@ -260,6 +260,13 @@ S2TC_API int s2tc_amd_serve(const s2tc_amd_job *jobs, int njobs, const s2tc_amd_
  * 0xffffffff restores); a low cap sends most blocks through the exact
  * rescan.  Call with no encode in flight. */
 S2TC_API int s2tc_amd_debug_set_scan_cap(unsigned cap);
+
+/* No counterpart in the reference; for tests only.  The waves of the
+ * Floyd-Steinberg dither wait for each other, each wait for at most so many
+ * looks (2^22, which 0xffffffff restores); a wait that ends without what it
+ * waited for makes the call (rgb565_image, tx_compress_dxtn) an error.  This
+ * sets the bound for the calling thread's later calls. */
+S2TC_API void s2tc_amd_debug_set_fs_polls(unsigned polls);
 
 #ifdef __cplusplus
 }

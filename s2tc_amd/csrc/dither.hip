@@ -636,7 +636,8 @@ static int run_simple(const uint8_t *src, long long n, int plain, void *scr, con
 // (:1437-1449), dither other than NONE and FLOYDSTEINBERG means SIMPLE
 // (:1419-1431).
 int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, int dither, void *d_out,
-                  void *d_scratch, hipStream_t st, const void *d_carry_in, void *d_carry_out, bool host_src)
+                  void *d_scratch, hipStream_t st, const void *d_carry_in, void *d_carry_out, bool host_src,
+                  const FsWait &fs)
 {
 	if (srccomps != 3) srccomps = 4;
 	if (alphabits != 1 && alphabits != 4) alphabits = 8;
@@ -652,7 +653,7 @@ int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, 
 	if (dither == DITHER_FLOYDSTEINBERG) {
 		if (d_carry_in || d_carry_out)
 			return set_error(S2TC_E_ARG, "the Floyd-Steinberg dither does not run in bands");
-		return launch_rgb565_fs(src, srccomps, w, h, alphabits, (uint8_t *)d_out, d_scratch, st);
+		return launch_rgb565_fs(src, srccomps, w, h, alphabits, (uint8_t *)d_out, d_scratch, st, fs);
 	}
 	const uint8_t *ci = (const uint8_t *)d_carry_in;
 	uint8_t *co = (uint8_t *)d_carry_out;

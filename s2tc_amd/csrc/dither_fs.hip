@@ -59,9 +59,12 @@ namespace s2tc {
 // the carries so that those loads, which are not used, stay inside.
 #define FS_PAD_WORDS (FS_STEP * ((FS_LAG + 2) / FS_STEP + 2 * FS_AHEAD + 2))
 
-// Upper bound of a wave's unsuccessful polls (seconds); a wave only waits for
-// waves with smaller tickets, which run, so it is never reached.
-#define FS_POLL_MAX (1 << 21)
+// A wave only waits for waves with smaller tickets, which run.  Should a wait
+// all the same last longer than FsWait::polls looks at memory or FS_LDS_POLLS
+// times as many at LDS (a microsecond and a tenth of one each), the wave takes
+// zeros for the missing sums, sets FsWait::gave_up, which makes the call an
+// error, and waits no more, so that every wave still ends.
+#define FS_LDS_POLLS 8
 
 struct FsDims {
 	int w;         // texels per row
@@ -69,6 +72,7 @@ struct FsDims {
 	int nb;        // its bands
 	int nslots;    // slots per band row (a multiple of FS_AHEAD)
 	int wc;        // carry words per band: w rounded up to FS_STEP
+	int polls;     // FsWait::polls
 };
 
 // Scratch of a slab: nplanes channel planes, the carries of its bands, two
@@ -80,6 +84,7 @@ struct FsScratch {
 	uint32_t *edge;      // [channel][2][wc]
 	uint32_t *zeros;     // [FS_STEP * FS_ZERO_GROUPS]
 	unsigned *tickets;   // [2]
+	uint32_t *gave_up;   // FsWait::gave_up
 };
 
 // One channel's quantizer of v = u + 2048: q = clamp(floor(u * scale + bias),
@@ -237,6 +242,11 @@ struct FsGroup {
 		for (int i = 1; i < 8; ++i) m = max(m, c[i]);
 		return m == NO_CARRY;
 	}
+	__device__ __forceinline__ void clear()
+	{
+#pragma unroll
+		for (int i = 0; i < 8; ++i) c[i] = 0u;
+	}
 };
 
 // What a wave's slots share.  The pointers move with the rounds of FS_AHEAD
@@ -255,7 +265,8 @@ struct FsWave {
 	float one;
 	FsRow st;
 	float prev7;
-	int polls;
+	int patience;          // FsDims::polls, 0 after a wait that gave up
+	uint32_t *gave_up;
 };
 
 // Slot u of the round at j0.  LIN, LOUT: the carries come from, go to LDS.  sv
@@ -272,11 +283,18 @@ __device__ __forceinline__ void fs_slot_step(FsWave &f, int j0, int u, uint4 &sv
 			// registers of its own, so that the common path waits for its
 			// own prefetch alone
 			FsGroup t;
+			int left = f.patience * (LIN ? FS_LDS_POLLS : 1);
+			bool miss;
 			do {
-				++f.polls;
 				if (!LIN) __builtin_amdgcn_s_sleep(1);
 				t.template load<LIN>(f.cin, f.lin, u);
-			} while (__any((int)t.missing()) && f.polls < FS_POLL_MAX);
+				miss = __any((int)t.missing());
+			} while (miss && --left > 0);
+			if (__builtin_expect(miss, 0)) {
+				t.clear();
+				f.patience = 0;
+				if (f.lane == 0) *f.gave_up = 1u;
+			}
 			g = t;
 		}
 	}
@@ -405,7 +423,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_fs_rows(FsDims d, int ch0, int n
 	         back;
 	f.st = FsRow{0.0f, 0.0f, 0.0f, 0.0f};
 	f.prev7 = 0.0f;
-	f.polls = 0;
+	f.patience = d.polls;
+	f.gave_up = s.gave_up;
 	// the band's last lane that matters does texel w (its sum drains) at this step
 	const int nj = (d.w + (out ? FS_LAG + 1 : 2 * lastrow)) / FS_STEP + 1;
 	if constexpr (WAVES == 1) {
@@ -529,10 +548,13 @@ static int fs_rows(const FsDims &d, int ch0, int nch, FsQuant k0, FsQuant k1, Fs
 }
 
 int launch_rgb565_fs(const uint8_t *src, int srccomps, int w, int h, int alphabits, uint8_t *out, void *d_scratch,
-                     hipStream_t st)
+                     hipStream_t st, const FsWait &wait)
 {
-	const FsDims full = fs_dims(w, h);
+	if (!wait.gave_up) return set_error(S2TC_E_ARG, "the Floyd-Steinberg dither needs a word for its waits");
+	FsDims full = fs_dims(w, h);
+	full.polls = (int)std::min(wait.polls, FS_POLLS);
 	FsScratch s;
+	s.gave_up = wait.gave_up;
 	uint8_t *p = (uint8_t *)d_scratch;
 	s.planes = (uint4 *)p;
 	p += fs_plane_bytes(full);

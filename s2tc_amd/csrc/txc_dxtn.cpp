@@ -104,11 +104,43 @@ struct Ctx {
 	HostBuf in_stage, host_out;
 	hipEvent_t stage_ev[kRing] = {};    // last upload out of each buffer of in_stage
 	hipEvent_t out_ev[kOutRing] = {};   // encoded bands
-	// per-block calls: one mapped pinned page that the kernel reads the block's
-	// texels from (offset 0) and writes its encoding to (offset 64)
-	uint8_t *blk_host = nullptr;
-	void *blk_dev = nullptr;
+	// one mapped pinned page: per-block calls, whose kernel reads the block's
+	// texels from it (offset 0) and writes its encoding to it (offset 64), and the
+	// word of FsWait (kPageGaveUp)
+	uint8_t *page = nullptr;
+	uint8_t *page_dev = nullptr;
+	int ensure_page()
+	{
+		if (page) return 0;
+		if (int r = hip_check(hipHostMalloc((void **)&page, 4096, hipHostMallocMapped), "hipHostMalloc")) return r;
+		const int r = hip_check(hipHostGetDevicePointer((void **)&page_dev, page, 0), "hipHostGetDevicePointer");
+		if (r) {
+			(void)hipHostFree(page);
+			page = nullptr;
+		}
+		return r;
+	}
 };
+static const size_t kPageGaveUp = 128;
+
+// Looks that a wait of the Floyd-Steinberg dither lasts at most (test hook).
+static thread_local unsigned t_fs_polls = FS_POLLS;
+
+// The waits of a call's dither: before its launch, and after its synchronize.
+static int fs_begin(Ctx *c, int dither, FsWait &wait)
+{
+	if (dither != DITHER_FLOYDSTEINBERG) return 0;
+	if (int r = c->ensure_page()) return r;
+	*(volatile uint32_t *)(c->page + kPageGaveUp) = 0;
+	wait.gave_up = (uint32_t *)(c->page_dev + kPageGaveUp);
+	wait.polls = t_fs_polls;
+	return 0;
+}
+static int fs_end(Ctx *c, int dither)
+{
+	if (dither != DITHER_FLOYDSTEINBERG || !*(volatile uint32_t *)(c->page + kPageGaveUp)) return 0;
+	return set_error(S2TC_E_HIP, "the Floyd-Steinberg dither's waves waited too long for each other");
+}
 
 // Whether the work that an event follows is done (a query that is not leaves no
 // error behind for the next launch to find).
@@ -426,8 +458,10 @@ static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, con
 	} else {
 		if (int r = c->q.ensure(n * 4)) return r;
 		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height, dither))) return r;
+		FsWait wait;
+		if (int r = fs_begin(c, dither, wait)) return r;
 		if (int r = launch_rgb565(d_src, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p, c->stream,
-		                          nullptr, nullptr, direct))
+		                          nullptr, nullptr, direct, wait))
 			return r;
 		a.src = c->q.p;
 		a.src_kind = S2TC_SRC_QUANTIZED;
@@ -437,7 +471,8 @@ static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, con
 		if (int r = hip_check(hipMemcpyAsync(c->host_out.data(), c->out.p, obytes, hipMemcpyDeviceToHost, c->stream),
 		                      "D2H"))
 			return r;
-	return hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+	if (int r = hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
+	return fs_end(c, dither);
 }
 
 // ---- per-block entry points of s2tc_encode_block_func ----
@@ -456,22 +491,14 @@ static void encode_one_block(unsigned char *out, const unsigned char *rgba, int 
 	}
 	if (w < 1 || h < 1 || w > 4 || h > 4) return;
 	const int bs = block_bytes(dxt);
-	int r = 0;
-	if (!c->blk_host) {
-		r = hip_check(hipHostMalloc((void **)&c->blk_host, 4096, hipHostMallocMapped), "hipHostMalloc");
-		if (!r) r = hip_check(hipHostGetDevicePointer(&c->blk_dev, c->blk_host, 0), "hipHostGetDevicePointer");
-		if (r && c->blk_host) {
-			(void)hipHostFree(c->blk_host);
-			c->blk_host = nullptr;
-		}
-	}
+	int r = c->ensure_page();
 	if (!r) {
 		// the block's rows, packed, where the kernel reads them over the bus
-		for (int y = 0; y < h; ++y) memcpy(c->blk_host + y * w * 4, rgba + (size_t)y * iw * 4, (size_t)w * 4);
+		for (int y = 0; y < h; ++y) memcpy(c->page + y * w * 4, rgba + (size_t)y * iw * 4, (size_t)w * 4);
 		// A one-block image whose only block has index bidx in the generator.
 		// The selection-time mode is kept: quick mode runs with nrandom < 0,
 		// MODE_NORMAL with max(nrandom, 0) extra candidates.
-		uint8_t *dev = (uint8_t *)c->blk_dev;
+		uint8_t *dev = c->page_dev;
 		EncodeArgs a{dev, dev + 64, S2TC_SRC_QUANTIZED, w, h, dxt, cd, fast ? -1 : (nrandom > 0 ? nrandom : 0),
 		             refine, 0, 0};
 		const char *sv = getenv("S2TC_RANDOM_SEED");
@@ -484,7 +511,7 @@ static void encode_one_block(unsigned char *out, const unsigned char *rgba, int 
 		fprintf(stderr, "s2tc: %s\n", s2tc_amd_last_error());
 		return;
 	}
-	memcpy(out, c->blk_host + 64, bs);
+	memcpy(out, c->page + 64, bs);
 }
 
 template <int DXT, int CD, int FAST, int REFINE>
@@ -597,10 +624,15 @@ void rgb565_image(unsigned char *out, const unsigned char *rgba, int w, int h, i
 	if (!r) r = c->q.ensure(n * 4);
 	if (!r) r = c->scratch.ensure(rgb565_scratch_bytes(w, h, (int)dither));
 	if (!r) r = upload(c, c->src.p, rgba, n * sc);
-	if (!r) r = launch_rgb565(c->src.p, sc, w, h, alphabits, (int)dither, c->q.p, c->scratch.p, c->stream);
+	FsWait wait;
+	if (!r) r = fs_begin(c, (int)dither, wait);
+	if (!r)
+		r = launch_rgb565(c->src.p, sc, w, h, alphabits, (int)dither, c->q.p, c->scratch.p, c->stream, nullptr, nullptr,
+		                  false, wait);
 	if (!r) r = hip_check(hipMemcpyAsync(out, c->q.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
 	if (!r) r = hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 	if (r) (void)hipStreamSynchronize(c->stream);
+	else r = fs_end(c, (int)dither);
 	if (r) fprintf(stderr, "s2tc: rgb565_image failed (%d): %s\n", r, s2tc_amd_last_error());
 }
 
@@ -620,6 +652,8 @@ s2tc_encode_block_func_t s2tc_encode_block_func(enum DxtMode dxt, ColorDistMode 
 }
 
 void s2tc_amd_set_block_index(unsigned int index) { t_block_index = index; }
+
+void s2tc_amd_debug_set_fs_polls(unsigned polls) { t_fs_polls = std::min(polls, FS_POLLS); }
 
 // ---- S2TC decoders (s2tc_libtxc_dxtn.cpp:35-140) ----
 
