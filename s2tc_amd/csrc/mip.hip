@@ -263,6 +263,13 @@ extern "C" int s2tc_amd_mip_chain(const void *d_src, int width, int height, void
 		return n;
 	}
 	const uint32_t *in = (const uint32_t *)d_src;
+	const uintptr_t s0 = (uintptr_t)d_src, d0 = (uintptr_t)d_levels;
+	const size_t bytes = (size_t)width * height * 4;
+	if (s0 != d0 && s0 < d0 + total && d0 < s0 + bytes) {
+		// a source where levels go: copied before any is written
+		if (int r = hip_check(hipMemcpyAsync(base, d_src, bytes, hipMemcpyDeviceToDevice, st), "D2D")) return r;
+		in = (const uint32_t *)base;
+	}
 	int w = width, h = height;
 	size_t off = 0;
 	for (int l0 = 0; l0 < n - 1; l0 += 6) {
@@ -271,7 +278,7 @@ extern "C" int s2tc_amd_mip_chain(const void *d_src, int width, int height, void
 		m.in = in;
 		m.w = w;
 		m.h = h;
-		if (l0 == 0 && d_src != d_levels) m.out[0] = (uint32_t *)base;
+		if (l0 == 0 && (const uint8_t *)in != base) m.out[0] = (uint32_t *)base;
 		const dim3 grid((unsigned)((w + 63) / 64), (unsigned)((h + 63) / 64));
 		for (int l = 1; l <= 6 && l0 + l < n; ++l) {
 			off += align256((size_t)w * h * 4);
