@@ -268,6 +268,12 @@ S2TC_API int s2tc_amd_debug_set_scan_cap(unsigned cap);
  * sets the bound for the calling thread's later calls. */
 S2TC_API void s2tc_amd_debug_set_fs_polls(unsigned polls);
 
+/* No counterpart in the reference; for tests only.  The Floyd-Steinberg dither
+ * takes less device scratch where there is no more, and is then slower.  Scratch
+ * above so many bytes counts as not there in the calling thread's later calls
+ * ((size_t)-1 restores). */
+S2TC_API void s2tc_amd_debug_set_fs_scratch_max(size_t bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -579,9 +579,9 @@ static size_t simple_scratch_bytes(long long n)
 	return (size_t)(nw * 65 * (4 + 2 + 4 + 8) + nw) * 4 + 256;
 }
 
-size_t rgb565_scratch_bytes(int w, int h, int dither)
+size_t rgb565_scratch_bytes(int w, int h, int dither, size_t fs_slab)
 {
-	if (dither == DITHER_FLOYDSTEINBERG) return rgb565_fs_scratch_bytes(w, h);
+	if (dither == DITHER_FLOYDSTEINBERG) return rgb565_fs_scratch_bytes(w, h, fs_slab);
 	return simple_scratch_bytes((long long)w * h);
 }
 
@@ -637,7 +637,7 @@ static int run_simple(const uint8_t *src, long long n, int plain, void *scr, con
 // (:1419-1431).
 int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, int dither, void *d_out,
                   void *d_scratch, hipStream_t st, const void *d_carry_in, void *d_carry_out, bool host_src,
-                  const FsWait &fs)
+                  const FsRun &fs)
 {
 	if (srccomps != 3) srccomps = 4;
 	if (alphabits != 1 && alphabits != 4) alphabits = 8;

@@ -60,9 +60,9 @@ namespace s2tc {
 #define FS_PAD_WORDS (FS_STEP * ((FS_LAG + 2) / FS_STEP + 2 * FS_AHEAD + 2))
 
 // A wave only waits for waves with smaller tickets, which run.  Should a wait
-// all the same last longer than FsWait::polls looks at memory or FS_LDS_POLLS
+// all the same last longer than FsRun::polls looks at memory or FS_LDS_POLLS
 // times as many at LDS (a microsecond and a tenth of one each), the wave takes
-// zeros for the missing sums, sets FsWait::gave_up, which makes the call an
+// zeros for the missing sums, sets FsRun::gave_up, which makes the call an
 // error, and waits no more, so that every wave still ends.
 #define FS_LDS_POLLS 8
 
@@ -72,7 +72,7 @@ struct FsDims {
 	int nb;        // its bands
 	int nslots;    // slots per band row (a multiple of FS_AHEAD)
 	int wc;        // carry words per band: w rounded up to FS_STEP
-	int polls;     // FsWait::polls
+	int polls;     // FsRun::polls
 };
 
 // Scratch of a slab: nplanes channel planes, the carries of its bands, two
@@ -84,7 +84,7 @@ struct FsScratch {
 	uint32_t *edge;      // [channel][2][wc]
 	uint32_t *zeros;     // [FS_STEP * FS_ZERO_GROUPS]
 	unsigned *tickets;   // [2]
-	uint32_t *gave_up;   // FsWait::gave_up
+	uint32_t *gave_up;   // FsRun::gave_up
 };
 
 // One channel's quantizer of v = u + 2048: q = clamp(floor(u * scale + bias),
@@ -486,12 +486,10 @@ __global__ __launch_bounds__(256) void k_fs_finish(const uint8_t *__restrict__ s
 
 // ---- host ----
 
-// The image is dithered in slabs of whole bands whose planes fit
-// FS_SLAB_BYTES; the wavefront drains between slabs, which a 4096-wide image
-// does every 15,000 rows.
-#define FS_SLAB_BYTES ((size_t)512 << 20)
-
-static FsDims fs_dims(int w, int h)
+// The image is dithered in slabs of whole bands whose planes fit FsRun::slab;
+// the wavefront drains between slabs, which a 4096-wide image does every 15,000
+// rows with FS_SLAB.
+static FsDims fs_dims(int w, int h, size_t slab)
 {
 	FsDims d{};
 	d.w = w;
@@ -499,7 +497,7 @@ static FsDims fs_dims(int w, int h)
 	d.nslots = d.wc / FS_STEP + (FS_LAG + 2) / FS_STEP;
 	d.nslots = (d.nslots + FS_AHEAD - 1) / FS_AHEAD * FS_AHEAD;
 	const size_t band = (size_t)4 * d.nslots * FS_ROWS * sizeof(uint4);
-	const long long cap = std::max<long long>(1, (long long)(FS_SLAB_BYTES / band));
+	const long long cap = std::max<long long>(1, (long long)(slab / band));
 	d.nb = (int)std::min<long long>(((long long)h + FS_ROWS - 1) / FS_ROWS, cap);
 	return d;
 }
@@ -512,9 +510,9 @@ static size_t fs_plane_bytes(const FsDims &d)
 static size_t fs_carry_bytes(const FsDims &d) { return fs_align(((size_t)4 * d.nb * d.wc + FS_PAD_WORDS) * 4); }
 static size_t fs_edge_bytes(const FsDims &d) { return fs_align(((size_t)8 * d.wc + FS_PAD_WORDS) * 4); }
 
-size_t rgb565_fs_scratch_bytes(int w, int h)
+size_t rgb565_fs_scratch_bytes(int w, int h, size_t slab)
 {
-	const FsDims d = fs_dims(w, h);
+	const FsDims d = fs_dims(w, h, slab);
 	return fs_plane_bytes(d) + fs_carry_bytes(d) + fs_edge_bytes(d) + 512;
 }
 
@@ -548,13 +546,13 @@ static int fs_rows(const FsDims &d, int ch0, int nch, FsQuant k0, FsQuant k1, Fs
 }
 
 int launch_rgb565_fs(const uint8_t *src, int srccomps, int w, int h, int alphabits, uint8_t *out, void *d_scratch,
-                     hipStream_t st, const FsWait &wait)
+                     hipStream_t st, const FsRun &run)
 {
-	if (!wait.gave_up) return set_error(S2TC_E_ARG, "the Floyd-Steinberg dither needs a word for its waits");
-	FsDims full = fs_dims(w, h);
-	full.polls = (int)std::min(wait.polls, FS_POLLS);
+	if (!run.gave_up) return set_error(S2TC_E_ARG, "the Floyd-Steinberg dither needs a word for its waits");
+	FsDims full = fs_dims(w, h, run.slab);
+	full.polls = (int)std::min(run.polls, FS_POLLS);
 	FsScratch s;
-	s.gave_up = wait.gave_up;
+	s.gave_up = run.gave_up;
 	uint8_t *p = (uint8_t *)d_scratch;
 	s.planes = (uint4 *)p;
 	p += fs_plane_bytes(full);

@@ -55,24 +55,29 @@ int launch_pull(void *dst, const void *src, size_t n, hipStream_t st);
 // states in d_carry_out for the next band.
 // host_src: d_src is pinned host memory, worth reading once only; d_out is then
 // 16-byte aligned.
-// fs: the waits of the Floyd-Steinberg dither's waves for each other.  gave_up, a
-// word in mapped pinned memory that the caller clears before, is 1 after the
-// launch if one of them ended without what it waited for, and the output is then
-// wrong; polls bounds each wait (FS_POLLS looks at memory take seconds).
+// fs: a run of the Floyd-Steinberg dither.  Its waves wait for each other:
+// gave_up, a word in mapped pinned memory that the caller clears before, is 1
+// after the launch if one of them ended without what it waited for, and the
+// output is then wrong; polls bounds each wait (FS_POLLS looks at memory take
+// seconds).  slab bounds the scratch for channel planes, of which one band of 64
+// rows is the least (512 bytes a column); less than the image needs costs the
+// time to drain and fill the wavefront between slabs.
 static const unsigned FS_POLLS = 1u << 22;
-struct FsWait {
+static const size_t FS_SLAB = (size_t)512 << 20;
+struct FsRun {
 	uint32_t *gave_up = nullptr;
 	unsigned polls = FS_POLLS;
+	size_t slab = FS_SLAB;
 };
-size_t rgb565_scratch_bytes(int w, int h, int dither);
+size_t rgb565_scratch_bytes(int w, int h, int dither, size_t fs_slab = FS_SLAB);
 int launch_rgb565(const void *d_src, int srccomps, int w, int h, int alphabits, int dither, void *d_out,
                   void *d_scratch, hipStream_t st, const void *d_carry_in = nullptr, void *d_carry_out = nullptr,
-                  bool host_src = false, const FsWait &fs = FsWait());
+                  bool host_src = false, const FsRun &fs = FsRun());
 
 // The Floyd-Steinberg dither (dither_fs.hip), arguments normalised.
-size_t rgb565_fs_scratch_bytes(int w, int h);
+size_t rgb565_fs_scratch_bytes(int w, int h, size_t slab);
 int launch_rgb565_fs(const uint8_t *src, int srccomps, int w, int h, int alphabits, uint8_t *out, void *d_scratch,
-                     hipStream_t st, const FsWait &wait);
+                     hipStream_t st, const FsRun &run);
 
 inline int block_bytes(int dxt) { return dxt == DXT1 ? 8 : 16; }
 

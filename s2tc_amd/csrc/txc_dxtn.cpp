@@ -41,6 +41,12 @@ struct DevBuf {
 		cap = n;
 		return 0;
 	}
+	void release()
+	{
+		if (p) (void)hipFree(p);
+		p = nullptr;
+		cap = 0;
+	}
 };
 
 // Pinned host memory (hipHostMalloc): staging for the host-buffer entry
@@ -106,7 +112,7 @@ struct Ctx {
 	hipEvent_t out_ev[kOutRing] = {};   // encoded bands
 	// one mapped pinned page: per-block calls, whose kernel reads the block's
 	// texels from it (offset 0) and writes its encoding to it (offset 64), and the
-	// word of FsWait (kPageGaveUp)
+	// word of FsRun (kPageGaveUp)
 	uint8_t *page = nullptr;
 	uint8_t *page_dev = nullptr;
 	int ensure_page()
@@ -127,13 +133,13 @@ static const size_t kPageGaveUp = 128;
 static thread_local unsigned t_fs_polls = FS_POLLS;
 
 // The waits of a call's dither: before its launch, and after its synchronize.
-static int fs_begin(Ctx *c, int dither, FsWait &wait)
+static int fs_begin(Ctx *c, int dither, FsRun &run)
 {
 	if (dither != DITHER_FLOYDSTEINBERG) return 0;
 	if (int r = c->ensure_page()) return r;
 	*(volatile uint32_t *)(c->page + kPageGaveUp) = 0;
-	wait.gave_up = (uint32_t *)(c->page_dev + kPageGaveUp);
-	wait.polls = t_fs_polls;
+	run.gave_up = (uint32_t *)(c->page_dev + kPageGaveUp);
+	run.polls = t_fs_polls;
 	return 0;
 }
 static int fs_end(Ctx *c, int dither)
@@ -231,8 +237,14 @@ static Ctx *ctx_acquire()
 	return c;
 }
 
+// Scratch that an idle context keeps: that of 4096 x 4096 with the
+// Floyd-Steinberg dither (134 MiB); to give back and to allocate more takes 0.27
+// ms, in calls of 5 ms and more.
+static const size_t kKeepScratch = (size_t)192 << 20;
+
 static void ctx_release(Ctx *c)
 {
+	if (c->scratch.cap > kKeepScratch) c->scratch.release();
 	std::lock_guard<std::mutex> lk(g_pool_mu);
 	g_pool.push_back(c);
 }
@@ -245,6 +257,34 @@ struct CtxGuard {
 		if (c) ctx_release(c);
 	}
 };
+
+// Scratch of a dither.  That of the Floyd-Steinberg dither is FsRun::slab and
+// somewhat more: where the device has not that much left, what idle contexts keep
+// is given back, and then the slabs get smaller, to one band of rows if need be.
+static thread_local size_t t_fs_scratch_max = ~(size_t)0;  // test hook
+
+static int dither_scratch(Ctx *c, int w, int h, int dither, FsRun &run)
+{
+	size_t n = rgb565_scratch_bytes(w, h, dither, run.slab);
+	if (dither != DITHER_FLOYDSTEINBERG) return c->scratch.ensure(n);
+	for (bool trimmed = false;;) {
+		const int r = n > t_fs_scratch_max ? set_error(S2TC_E_HIP, "no scratch of %zu bytes", n) : c->scratch.ensure(n);
+		if (!r) return 0;
+		(void)hipGetLastError();  // not for the next launch to find
+		if (!trimmed) {
+			std::lock_guard<std::mutex> lk(g_pool_mu);
+			for (Ctx *idle : g_pool) idle->scratch.release();
+			trimmed = true;
+			continue;
+		}
+		const size_t before = n;
+		while (n == before) {
+			if (!run.slab) return r;
+			run.slab /= 4;
+			n = rgb565_scratch_bytes(w, h, dither, run.slab);
+		}
+	}
+}
 
 // Environment configuration of s2tc_libtxc_dxtn.cpp:156-216.
 struct EnvConfig {
@@ -457,11 +497,11 @@ static int encode_host_image_on(Ctx *c, int srccomps, int width, int height, con
 		a.src_kind = S2TC_SRC_RGBA8;
 	} else {
 		if (int r = c->q.ensure(n * 4)) return r;
-		if (int r = c->scratch.ensure(rgb565_scratch_bytes(width, height, dither))) return r;
-		FsWait wait;
-		if (int r = fs_begin(c, dither, wait)) return r;
+		FsRun run;
+		if (int r = fs_begin(c, dither, run)) return r;
+		if (int r = dither_scratch(c, width, height, dither, run)) return r;
 		if (int r = launch_rgb565(d_src, srccomps, width, height, alphabits, dither, c->q.p, c->scratch.p, c->stream,
-		                          nullptr, nullptr, direct, wait))
+		                          nullptr, nullptr, direct, run))
 			return r;
 		a.src = c->q.p;
 		a.src_kind = S2TC_SRC_QUANTIZED;
@@ -622,13 +662,13 @@ void rgb565_image(unsigned char *out, const unsigned char *rgba, int w, int h, i
 	const size_t n = (size_t)w * h;
 	int r = c->src.ensure(n * sc);
 	if (!r) r = c->q.ensure(n * 4);
-	if (!r) r = c->scratch.ensure(rgb565_scratch_bytes(w, h, (int)dither));
+	FsRun run;
+	if (!r) r = fs_begin(c, (int)dither, run);
+	if (!r) r = dither_scratch(c, w, h, (int)dither, run);
 	if (!r) r = upload(c, c->src.p, rgba, n * sc);
-	FsWait wait;
-	if (!r) r = fs_begin(c, (int)dither, wait);
 	if (!r)
 		r = launch_rgb565(c->src.p, sc, w, h, alphabits, (int)dither, c->q.p, c->scratch.p, c->stream, nullptr, nullptr,
-		                  false, wait);
+		                  false, run);
 	if (!r) r = hip_check(hipMemcpyAsync(out, c->q.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
 	if (!r) r = hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 	if (r) (void)hipStreamSynchronize(c->stream);
@@ -654,6 +694,8 @@ s2tc_encode_block_func_t s2tc_encode_block_func(enum DxtMode dxt, ColorDistMode 
 void s2tc_amd_set_block_index(unsigned int index) { t_block_index = index; }
 
 void s2tc_amd_debug_set_fs_polls(unsigned polls) { t_fs_polls = std::min(polls, FS_POLLS); }
+
+void s2tc_amd_debug_set_fs_scratch_max(size_t bytes) { t_fs_scratch_max = bytes; }
 
 // ---- S2TC decoders (s2tc_libtxc_dxtn.cpp:35-140) ----
 
