@@ -526,6 +526,17 @@ S2TC_D uint32_t alpha_refine_group(int a, bool valid, int refine, int &a0, int &
 	return idx;
 }
 
+// Orders the group memory accesses of a block's lanes, which are lanes of one
+// wave: what one of them wrote before, the others read after.  No barrier, so it
+// may stand in a branch that the four blocks of a workgroup take differently,
+// where __syncthreads() may not.
+S2TC_D void block_sync()
+{
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // x % l for x < 2^31 and 1 <= l <= 256 by a multiplier m in [2^32 / l - 2,
 // 2^32 / l]: mul_hi falls short of x / l by less than 1 before its floor, so it
 // is the quotient or one less, and the remainder, below 2 l, only needs the low
@@ -634,7 +645,7 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 			ul = (uint32_t *)(sm.rows + cap - 3 * m);
 			if (dd)
 				for (int z = t; z < V; z += 16) T1[z] = T2[z] = 0x7fffffff;
-			__syncthreads();
+			block_sync();
 		}
 		// candidate i of cell z: the first two indices of every cell
 		const auto enter = [&](int z, int i) {
@@ -679,7 +690,7 @@ S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int 
 		if (use) sm.cand[pos] = v | ((uint32_t)alpha << 16);
 		if (none && t == 0) sm.cand[0] = 0u;
 		if (n == 1) {  // "hack for last miplevel" (:996-1001); ca[1] pinned to 0
-			__syncthreads();
+			block_sync();
 			if (t == 0) sm.cand[1] = sm.cand[0] & 0xffffu;
 			n = m = 2;
 		}
