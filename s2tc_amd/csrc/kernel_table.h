@@ -35,7 +35,7 @@ struct KernelTable {
 	int normal_smem_cand;         // LDS bytes per candidate slot of a 4-block workgroup (candidate words)
 	int normal_smem_fixed;        // plus these bytes (features of the 16 texel candidates of 4 blocks)
 	const void *fast_batch[3][3]; // [dxt][refine]: persistent quick-mode kernel over a job list
-	const void *normal_batch;     // persistent MODE_NORMAL kernel over a job list
+	const void *normal_batch[2];  // [many]: persistent MODE_NORMAL kernel over a job list (many: class_many; null where never)
 	const void *normal_batch_wide;  // the same with group memory in global scratch
 	const void *all16[3][2];      // [dxt][raw]: MODE_NORMAL without random colours, one lane per block
 	const void *all16_batch[3][3];  // [dxt][refine]: its persistent batch form
@@ -55,15 +55,23 @@ struct KernelTable {
 // 278 us and 1075 -> 975 us.  Outside that range, and where a launch has no
 // more workgroups than eight to a CU, the third row block only costs moves:
 // 48 random colours up to 8% slower, 128 SRGB 2%, 256 x 256 SRGB 8%.
-// The batch kernel always has two: its class takes textures of all counts, and
-// 40 textures of 256 x 256 with 8 random colours beside one with 64 took 401 us
-// with two and 456 us with three (SRGB), 40 with 64 1314 and 1350 us; RGB, YUV
-// and SRGB_MIXED alike, and the other distances gain nothing.
 #define S2TC_RB_FEW 2
 #define S2TC_RB_MANY 3
 inline bool normal_many(int pbw, long long workgroups)
 {
 	return pbw >= 5 && pbw <= 8 && workgroups > 8 * 256;
+}
+
+// A class of a batch takes textures of all counts: three row blocks where three
+// quarters of its pair work (blocks times row blocks squared) lie in that range.
+// Measured (40 textures of 256 x 256 with few random colours and some with 64,
+// the class alone, two and three): SRGB 8 and one 64 401 and 456 us, 16 and ten
+// 64 697 and 760 us; NORMALMAP alike with both; only 64: SRGB 1314 and 1350 us,
+// NORMALMAP within 1%.  Beside other classes three are the faster ones for them:
+// 120 textures of the serving mix, every random one with 64, 1.69 and 1.53 ms.
+inline bool class_many(double many_work, double work, int pbw_max, long long workgroups)
+{
+	return normal_many(pbw_max, workgroups) && 4 * many_work >= 3 * work;
 }
 
 #if defined(__HIP__) || defined(__HIPCC__)

