@@ -57,9 +57,9 @@ struct KernelTable {
 // 48 random colours up to 8% slower, 128 SRGB 2%, 256 x 256 SRGB 8%.
 #define S2TC_RB_FEW 2
 #define S2TC_RB_MANY 3
-inline bool normal_many(int pbw, long long workgroups)
+inline bool normal_many(int pbw, long long workgroups, int cus)
 {
-	return pbw >= 5 && pbw <= 8 && workgroups > 8 * 256;
+	return pbw >= 5 && pbw <= 8 && workgroups > 8LL * cus;
 }
 
 // A class of a batch takes textures of all counts: three row blocks where three
@@ -69,9 +69,9 @@ inline bool normal_many(int pbw, long long workgroups)
 // 64 697 and 760 us; NORMALMAP alike with both; only 64: SRGB 1314 and 1350 us,
 // NORMALMAP within 1%.  Beside other classes three are the faster ones for them:
 // 120 textures of the serving mix, every random one with 64, 1.69 and 1.53 ms.
-inline bool class_many(double many_work, double work, int pbw_max, long long workgroups)
+inline bool class_many(double many_work, double work, int pbw_max, long long workgroups, int cus)
 {
-	return normal_many(pbw_max, workgroups) && 4 * many_work >= 3 * work;
+	return normal_many(pbw_max, workgroups, cus) && 4 * many_work >= 3 * work;
 }
 
 #if defined(__HIP__) || defined(__HIPCC__)

@@ -10,15 +10,13 @@ namespace s2tc {
 
 int device_cu_count()
 {
-	static int ncu = 0;
-	if (!ncu) {
+	static const int ncu = [] {
 		int dev = 0;
 		(void)hipGetDevice(&dev);
 		hipDeviceProp_t prop;
-		ncu = (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-		          ? prop.multiProcessorCount
-		          : 256;
-	}
+		return hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0 ? prop.multiProcessorCount
+		                                                                                        : 256;
+	}();
 	return ncu;
 }
 
@@ -101,7 +99,7 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 		const int pbw = normal_pbw(d.nrandom);
 		c.pbw_max = std::max(c.pbw_max, pbw);
 		c.pair_work += (double)nb * pbw * pbw;
-		if (normal_many(pbw, INT_MAX)) c.many_work += (double)nb * pbw * pbw;
+		if (normal_many(pbw, INT_MAX, 1)) c.many_work += (double)nb * pbw * pbw;
 		c.jobs.push_back(d);
 		c.job_index.push_back(i);
 		// rough cost: quick mode ~1 per block, MODE_NORMAL ~ candidate pairs
@@ -112,7 +110,7 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 	for (auto &c : classes) {
 		const KernelTable &kt = kernel_table(c.cd);
 		c.ntiles = (int)((c.nblocks + c.tile - 1) / c.tile);
-		const bool many = kt.normal_batch[1] && class_many(c.many_work, c.pair_work, c.pbw_max, c.ntiles);
+		const bool many = kt.normal_batch[1] && class_many(c.many_work, c.pair_work, c.pbw_max, c.ntiles, device_cu_count());
 		c.kernel = c.wide     ? kt.normal_batch_wide
 		           : c.normal ? kt.normal_batch[many]
 		           : c.all16  ? kt.all16_batch[c.dxt][c.refine]

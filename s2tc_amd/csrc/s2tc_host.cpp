@@ -162,7 +162,7 @@ int launch_encode(const EncodeArgs &a, hipStream_t stream, void *ext_scratch, si
 	unsigned block_base = a.block_index_base;
 	if (nrandom <= S2TC_LDS_NRANDOM) {
 		dim3 grid((unsigned)((nb + 3) / 4));
-		const bool many = normal_many(pbw, grid.x);
+		const bool many = normal_many(pbw, grid.x, device_cu_count());
 		size_t smem = normal_group_smem(kt, pbw, many);
 		void *args[] = {(void *)&src, (void *)&width, (void *)&height, (void *)&dst, (void *)&dxt,
 		                (void *)&nrandom, (void *)&refine, (void *)&seed, (void *)&pbw, (void *)&block_base};

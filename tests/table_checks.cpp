@@ -36,10 +36,17 @@ int main()
 	} classes[] = {{3, 0, 40, true}, {2, 40, 1, false}, {2, 40, 10, false}, {4, 40, 1, false}, {3, 4, 40, true}};
 	for (const auto &c : classes) {
 		const double m = work(5, c.nmany), all = m + work(c.few, c.nfew);
-		if (class_many(m, all, 5, 1 << 20) != c.many || class_many(m, all, 5, 100) || class_many(m, all, 9, 1 << 20)) {
+		if (class_many(m, all, 5, 1 << 20, 256) != c.many || class_many(m, all, 5, 100, 256) ||
+		    class_many(m, all, 9, 1 << 20, 256)) {
 			printf("class of %d textures with %d row blocks and %d with 5\n", c.nfew, c.few, c.nmany);
 			return 1;
 		}
+	}
+	// more workgroups than eight to a CU of the device, however many it has
+	if (normal_many(5, 8 * 256, 256) || !normal_many(5, 8 * 256 + 1, 256) || normal_many(5, 256, 32) ||
+	    !normal_many(5, 257, 32)) {
+		printf("workgroups per CU\n");
+		return 1;
 	}
 	printf("ok\n");
 	return 0;
