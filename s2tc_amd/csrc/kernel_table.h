@@ -35,7 +35,7 @@ struct KernelTable {
 	int normal_smem_cand;         // LDS bytes per candidate slot of a 4-block workgroup (candidate words)
 	int normal_smem_fixed;        // plus these bytes (features of the 16 texel candidates of 4 blocks)
 	const void *fast_batch[3][3]; // [dxt][refine]: persistent quick-mode kernel over a job list
-	const void *normal_batch[2];  // [many]: persistent MODE_NORMAL kernel over a job list (many: class_many; null where never)
+	const void *normal_batch[2];  // [many]: persistent MODE_NORMAL kernel over a job list (many: class_many)
 	const void *normal_batch_wide;  // the same with group memory in global scratch
 	const void *all16[3][2];      // [dxt][raw]: MODE_NORMAL without random colours, one lane per block
 	const void *all16_batch[3][3];  // [dxt][refine]: its persistent batch form
@@ -66,9 +66,10 @@ inline bool normal_many(int pbw, long long workgroups, int cus)
 // quarters of its pair work (blocks times row blocks squared) lie in that range.
 // Measured (40 textures of 256 x 256 with few random colours and some with 64,
 // the class alone, two and three): SRGB 8 and one 64 401 and 456 us, 16 and ten
-// 64 697 and 760 us; NORMALMAP alike with both; only 64: SRGB 1314 and 1350 us,
-// NORMALMAP within 1%.  Beside other classes three are the faster ones for them:
-// 120 textures of the serving mix, every random one with 64, 1.69 and 1.53 ms.
+// 64 697 and 760 us; NORMALMAP alike with both.  Only 64 random colours, 4
+// workgroups a CU: RGB 5% slower with three, SRGB 2%, the others within 1%; but
+// with as many as fit a CU, as in a tuned batch, faster: the YUV class of the
+// serving pool 2.88 and 2.12 ms, the pool as one batch 4.56 and 3.97 ms.
 inline bool class_many(double many_work, double work, int pbw_max, long long workgroups, int cus)
 {
 	return normal_many(pbw_max, workgroups, cus) && 4 * many_work >= 3 * work;
@@ -84,7 +85,9 @@ inline bool class_many(double many_work, double work, int pbw_max, long long wor
 // the other rows.  With three in registers and five in all, 560 instead of
 // 512, so that the tables of the scan over distinct colours hold a box of 160
 // cells (two ints a cell, three a candidate): 80 candidates fall on 63 of
-// them, a row block less, and twelve workgroups still fit a CU.
+// them, a row block less, and twelve workgroups still fit a CU.  Measured: a 4096 x
+// 4096 normal map with 64 random colours 499 -> 491 us; 1024 x 1024 with 49 to 64
+// under five distances and three contents within 1.5% either way, 1.000 on average.
 S2TC_HD inline int normal_row_ints(int pbw, int rb)
 {
 	const int rows = 256 * (pbw > rb ? pbw - rb : 0);

@@ -249,6 +249,9 @@ S2TC_D void normal_image_tile(const uint32_t *__restrict__ src, int width, int h
 // textures of 256 x 256, 16 random colours: RGB 327 us, 277 us without).  Three
 // waves; RGB and YUV with two row blocks in the registers that they take by
 // themselves (told of three, they come out 4% slower, the others up to 2% faster).
+// With three row blocks some scratch is left under RGB, YUV, SRGB and SRGB_MIXED
+// (36 to 76 bytes); two waves without it cost the serving pool 12% (as one batch
+// on four streams, 4 workgroups a CU: 4.71 and 5.34 ms).
 #define S2TC_ALONE(CD, RB) (RB == S2TC_RB_FEW && CD <= CD_YUV)
 #define S2TC_BATCH_WAVES(CD, RB) __attribute__((amdgpu_waves_per_eu(S2TC_ALONE(CD, RB) ? 1 : 3, S2TC_ALONE(CD, RB) ? 8 : 3)))
 
@@ -657,11 +660,7 @@ extern "C" void S2TC_CAT(s2tc_kernels_cd, S2TC_CD)(KernelTable *kt)
 	for (int d = 0; d < 3; ++d) kt->fast_batch[d][0] = kt->fast_batch[d][1] = kt->fast_batch[d][2] = nullptr;
 #endif
 	kt->normal_batch[0] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_FEW>;
-#if S2TC_CD == 2 || S2TC_CD >= 4
 	kt->normal_batch[1] = (const void *)k_normal_batch<S2TC_CD, S2TC_RB_MANY>;
-#else  /* RGB, YUV, SRGB_MIXED: 76 bytes a lane in scratch, and 5 to 12% slower alone */
-	kt->normal_batch[1] = nullptr;
-#endif
 	kt->normal_batch_wide = (const void *)k_normal_batch_wide<S2TC_CD>;
 	kt->error[DXT1][0] = (const void *)k_colordist_error<S2TC_CD, DXT1, false>;
 	kt->error[DXT3][0] = (const void *)k_colordist_error<S2TC_CD, DXT3, false>;

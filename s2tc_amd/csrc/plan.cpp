@@ -110,7 +110,7 @@ int plan_classes(const s2tc_amd_job *jobs, int njobs, std::vector<ClassPlan> &cl
 	for (auto &c : classes) {
 		const KernelTable &kt = kernel_table(c.cd);
 		c.ntiles = (int)((c.nblocks + c.tile - 1) / c.tile);
-		const bool many = kt.normal_batch[1] && class_many(c.many_work, c.pair_work, c.pbw_max, c.ntiles, device_cu_count());
+		const bool many = class_many(c.many_work, c.pair_work, c.pbw_max, c.ntiles, device_cu_count());
 		c.kernel = c.wide     ? kt.normal_batch_wide
 		           : c.normal ? kt.normal_batch[many]
 		           : c.all16  ? kt.all16_batch[c.dxt][c.refine]

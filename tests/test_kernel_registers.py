@@ -1,6 +1,6 @@
 """Registers of the built kernels, from the metadata of the library's gfx950 code objects: the random-candidate
-encoders keep everything in registers and LDS, none in scratch memory (but for 36 bytes a lane of the SRGB batch
-kernel with three row blocks in registers, which is the faster one with them)."""
+encoders keep everything in registers and LDS, none in scratch memory (but for up to 76 bytes a lane of the batch kernel
+with three row blocks in registers, which costs it less than the waves that it would give up)."""
 import os
 import re
 import struct
@@ -47,5 +47,5 @@ def test_random_candidate_kernels_use_no_scratch(tmp_path):
         pytest.skip("library or llvm-readelf not here")
     kernels = {k: v for k, v in _kernels(tmp_path).items() if "k_normal" in k}
     assert sum("14k_normal_batchI" in k for k in kernels) >= 8 and sum("8k_normalI" in k for k in kernels) >= 16
-    over = {k: v for k, v in kernels.items() if v > (36 if "14k_normal_batchILi2ELi3E" in k else 0)}
+    over = {k: v for k, v in kernels.items() if v > (76 if re.search("14k_normal_batchILi.ELi3E", k) else 0)}
     assert over == {}
