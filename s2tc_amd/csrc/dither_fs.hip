@@ -26,10 +26,14 @@
 // KiB); a step's quantized values go back into the first half of their slot,
 // and a last kernel interleaves the channels.
 //
-// Measured (MI355X, RGBA, alpha copied): 1024 x 1024 0.19 ms, 4096 x 4096 0.80
-// ms, of which k_fs_rows 47 ns a step; one workgroup per channel with a
-// barrier per step took 2.3 ms and 37 ms.  Carries through global memory
-// alone: 0.21 and 0.89 ms.
+// Measured (MI355X, RGBA, alpha copied): 1024 x 1024 0.22 ms, 4096 x 4096 0.80
+// ms; k_fs_rows takes 68 ns a step at 1024 x 1024 (209 us; the alpha pass with one
+// channel 56 ns, 174 us), where the waves of each band still start up for much of
+// the time, and 47 ns at 4096 x 4096.  One workgroup per channel with a barrier per
+// step took 2.3 ms and 37 ms; carries through global memory alone 0.21 and 0.89 ms.
+//
+// Memory: the planes take 8 bytes a texel and a band of 64 rows 512 a column and
+// 80 KiB, in slabs of up to FS_SLAB; rows of a few texels are padded to 160 steps.
 //
 // The reference reuses one error buffer for the colour and the alpha pass and
 // does not clear the part the alpha pass reads for its first row: that row
@@ -51,7 +55,7 @@ namespace s2tc {
 #define FS_AHEAD 4              // slots loaded ahead of the one in work
 #define FS_ZERO_GROUPS (2 * FS_AHEAD)  // zeros read by the lanes that get no carries
 #define FS_WAVES 4              // bands of a workgroup: one wave on each SIMD of a CU
-#define FS_LDS_MAX (156 << 10)  // widest rows whose carries fit LDS: 13,300 texels
+#define FS_LDS_MAX (156 << 10)  // LDS of a workgroup: rows of up to FS_LDS_WIDTH texels
 #define NO_CARRY 0xffffffffu    // a carry word that is not there yet (a NaN)
 
 // A wave's last slot lies at most FS_LAG steps and a round of FS_AHEAD after
@@ -547,6 +551,16 @@ __global__ __launch_bounds__(64) void k_fs_small(const uint8_t *__restrict__ src
 
 // ---- host ----
 
+// LDS bytes of a workgroup of FS_WAVES waves for rows of wc carry words, and the
+// widest rows whose carries fit.
+static constexpr size_t fs_lds_bytes(int wc)
+{
+	return (size_t)FS_LDS_CARRY * 8 + ((size_t)(FS_WAVES - 1) * wc + FS_PAD_WORDS) * 4;
+}
+#define FS_LDS_WIDTH 13216
+static_assert(fs_lds_bytes(FS_LDS_WIDTH) <= FS_LDS_MAX && fs_lds_bytes(FS_LDS_WIDTH + FS_STEP) > FS_LDS_MAX,
+              "FS_LDS_WIDTH");
+
 // The image is dithered in slabs of whole bands whose planes fit FsRun::slab;
 // the wavefront drains between slabs, which a 4096-wide image does every 15,000
 // rows with FS_SLAB.
@@ -589,8 +603,8 @@ static FsQuant fs_quant(int shift)
 static int fs_rows(const FsDims &d, int ch0, int nch, FsQuant k0, FsQuant k1, FsQuant k2, const FsScratch &s,
                    int ticket, int edge_in, int has_next, int last_red, hipStream_t st)
 {
-	const size_t lds = (size_t)FS_LDS_CARRY * 8 + ((size_t)(FS_WAVES - 1) * d.wc + FS_PAD_WORDS) * 4;
-	if (lds > FS_LDS_MAX) {
+	const size_t lds = fs_lds_bytes(d.wc);
+	if (d.wc > FS_LDS_WIDTH) {
 		k_fs_rows<1><<<(unsigned)(d.nb * nch), 64, 0, st>>>(d, ch0, nch, k0, k1, k2, s, ticket, edge_in, has_next,
 		                                                    last_red);
 	} else {
