@@ -585,7 +585,7 @@ template <int CD> struct PlainScan {
 // list is the count of cells with an earlier first index; up to 8 colours in
 // all four blocks, the rows are held twice and four rotations do.  The kernel
 // is bound by vector instructions.  Measured (MI355X, 4096 x 4096 smooth normal
-// map, 64 random colours, LOOP): 501 us, 802 us with three passes over the
+// map, 64 random colours, LOOP): 491 us, 802 us with three passes over the
 // candidates for the list and two register row blocks.
 template <int CD, int RB, bool DEDUP, bool CLEAR = false>
 S2TC_D void encode_block_normal(uint32_t tex, int t, int w, int h, int dxt, int nrandom, int refine, uint32_t bkey,
